@@ -257,7 +257,7 @@ __device__ inline int load_vector_lanes(const int32_t* p, int lane_zero) {
 // page.  The page id is wave-uniform (scalar load) and each block gets a buffer
 // descriptor covering only its valid rows: rows past `lim` read as zero without a
 // memory request, and no access can leave the block.
-// GenericPager: any other page size, per-lane table lookups and predicated loads.
+// GenericPager: any other page size, a pool row per token.
 // ---------------------------------------------------------------------------------
 struct TileRegs {
   u32x4 k[2][4];  // k[b][kk]: K row (block b, token c), dims 32kk + 8g .. +8
@@ -542,7 +542,15 @@ struct Lines : Base {
 
 // Pagers that load the K-operand layout into registers need nothing before the compute.
 template <class Pager, class Raw>
-__device__ inline void ready_tile(const Pager&, Raw&) {}
+__device__ inline void ready_tile(const Pager&, Raw&, int) {}
+
+// The last tile of a range is computed with no further tile's loads behind it.
+template <class Pager>
+__device__ inline void last_tile(const Pager&) {}
+template <class Base, int SLABS>
+__device__ inline void last_tile(const Lines<Base, SLABS>&) {
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // K in the slab; 8 V loads may remain
+}
 
 // The tile's K rows have reached the slab once its 8 K loads are done.  Vector memory
 // loads complete in order, and at least 8 were issued after them (the tile's V loads),
@@ -552,7 +560,7 @@ __device__ inline void ready_tile(const Pager&, Raw&) {}
 // barrier, so the slab's reads stay below it; consumed by the tile's MFMAs, they are
 // done before the slab's next loads are issued.
 template <class Base, int SLABS>
-__device__ inline void ready_tile(const Lines<Base, SLABS>& pg, LineTile& r) {
+__device__ inline void ready_tile(const Lines<Base, SLABS>& pg, LineTile& r, int) {
   const int c = pg.lane & 15, g = pg.lane >> 4;
   if constexpr (SLABS == 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
   else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
@@ -626,59 +634,110 @@ struct Fp8Pager {
   }
 };
 
+// Pager for page sizes that are not multiples of 16: a 16-token block may span pages, so
+// each token row has an address of its own.
+//   - Table entries are loaded 64 at a time (lane l: entry base + l), the next 64 one window
+//     ahead, so a tile's lookups wait for no memory: a vector load of a tile's entries two
+//     tiles ahead would return in order behind the K/V loads issued before it, and waiting
+//     for it would drain them.
+//   - Lane l forms the pool row of token l % 32 (one division per tile); the operand lanes
+//     take their rows from it by ds_bpermute, two for K and eight for V.
+//   - Tokens at or past `lim` take the last valid token's row: every load is in bounds with
+//     no branch around it.  Their scores are masked in compute_tile; their V (last tile
+//     only) reads as zero.
+// What bounds it: the tile's address work (~130 vector instructions) beside its loads, and
+// the longest row's units.  Measured on 16 rows of 100-6000 tokens, 4 KV heads, G = 8, bf16,
+// pages of 8, 4 splits (93 MB): 68.8 us per call with per-lane lookups and a branch around
+// each load, which waited for every lookup in turn; 44.4 us with the address work hoisted but
+// table loads and partial tiles still branched; 31.1 us without a branch in the loop.
 struct GenericPager {
   struct Pages {
-    long k[2];  // byte offset of this lane's K chunk per block, or -1
-    long v[8];  // byte offset of this lane's V chunk per slot, or -1
+    uint32_t k[2];  // pool row (head 0) of this lane's K token per block
+    uint32_t v[8];  // pool row of this lane's V token per slot
   };
   using Raw = TileRegs;
   const DecodeArgs& a;
   const int32_t* trow;
-  int lim;
-  long head_bytes, page_bytes;
-  int c, g;
+  int lim, lane;
+  const uint8_t* kbase;  // row 0 of this KV head
+  const uint8_t* vbase;
+  mutable int base;      // first page of the window: `cur` holds entries [base, base + 64),
+  mutable int cur, nxt;  // `nxt` [base + 64, base + 128), one per lane
 
-  __device__ GenericPager(const DecodeArgs& args, int row, int kvh, int limit, int lane)
-      : a(args), lim(limit) {
+  __device__ GenericPager(const DecodeArgs& args, int row, int kvh, int limit, int lane_id)
+      : a(args), lim(limit), lane(lane_id) {
     trow = a.block_table + (long)row * a.max_pages;
-    head_bytes = (long)kvh * a.page_size * (kD * 2);
-    page_bytes = (long)a.hkv * a.page_size * (kD * 2);
-    c = lane & 15;
-    g = lane >> 4;
+    const long head_bytes = (long)kvh * a.page_size * (kD * 2);
+    kbase = a.k_pages + head_bytes;
+    vbase = a.v_pages + head_bytes;
   }
-  __device__ inline long row_offset(int token) const {
-    if (token >= lim) return -1;
+  __device__ inline int load_entries(int first) const {
+    const int i = first + lane;
+    return trow[i < a.max_pages ? i : a.max_pages - 1];
+  }
+  __device__ inline int first_page(int tile) const {
     int logical, in_page;
-    page_of(a, token, logical, in_page);
-    const int page = clamp_page(a, trow[logical]);
-    return (long)page * page_bytes + head_bytes + (long)in_page * (kD * 2);
+    page_of(a, tile * kTile, logical, in_page);
+    return uniform(logical);
+  }
+  // Starts the window at tile t0; lookups then ascend one tile at a time.
+  __device__ inline void begin(int t0) const {
+    base = first_page(t0);
+    cur = load_entries(base);
+    nxt = load_entries(base + 64);
   }
   __device__ inline Pages lookup(int tile) const {
+    int token = tile * kTile + (lane & 31), logical, in_page;
+    token = token < lim ? token : lim - 1;
+    page_of(a, token, logical, in_page);
+    const int i = logical - base;
+    const int lo = __builtin_amdgcn_ds_bpermute(4 * i, cur), hi = __builtin_amdgcn_ds_bpermute(4 * i, nxt);
+    const int page = clamp_page(a, i < 64 ? lo : hi);
+    const uint32_t row = (uint32_t)page * (uint32_t)(a.hkv * a.page_size) + (uint32_t)in_page;
+    const int c = lane & 15, g = lane >> 4;
     Pages p;
-    const int tok0 = tile * kTile;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const long o = row_offset(tok0 + b * 16 + c);
-      p.k[b] = o < 0 ? -1 : o + g * 16;
-    }
+    for (int b = 0; b < 2; ++b) p.k[b] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (b * 16 + c), (int)row);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const long o = row_offset(tok0 + v_slot_token(g, j));
-      p.v[j] = o < 0 ? -1 : o + c * 16;
-    }
+    for (int j = 0; j < 8; ++j)
+      p.v[j] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * v_slot_token(g, j), (int)row);
+    // The window moves on after its last use (a tile spans at most 32 pages, so the next
+    // tile lies within two windows of this one).  The second window is loaded anew for
+    // every tile, ahead of the next tile's K/V loads (no branch, as in issue).
+    const bool move = first_page(tile + 1) >= base + 64;
+    base = move ? base + 64 : base;
+    cur = move ? nxt : cur;
+    nxt = load_entries(base + 64);
     return p;
   }
+  __device__ static inline u32x4 load_nt(const uint8_t* p) {
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4*)p);
+  }
+  // Always 16 loads, with no branch: the compiler then knows how many were issued after a
+  // table load and waits for no more than it must.
   __device__ inline void issue(int, const Pages& p, TileRegs& r) const {
-    const u32x4 z = {0u, 0u, 0u, 0u};
+    const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 2; ++b) {
+      const uint8_t* src = kbase + (uint64_t)p.k[b] * (kD * 2) + g * 16;
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        r.k[b][kk] = p.k[b] < 0 ? z : *(const u32x4*)(a.k_pages + p.k[b] + kk * 64);
+      for (int kk = 0; kk < 4; ++kk) r.k[b][kk] = load_nt(src + kk * 64);
+    }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) r.v[j] = p.v[j] < 0 ? z : *(const u32x4*)(a.v_pages + p.v[j]);
+    for (int j = 0; j < 8; ++j) r.v[j] = load_nt(vbase + (uint64_t)p.v[j] * (kD * 2) + c * 16);
   }
 };
+
+// V of the tokens past the range reads as zero (their weights are 0, but 0 x NaN is not);
+// selected for every tile, as a branch around loaded registers costs the loop its loads in
+// flight.
+__device__ inline void ready_tile(const GenericPager& pg, TileRegs& r, int tile) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t keep = tile * kTile + v_slot_token(pg.lane >> 4, j) < pg.lim ? ~0u : 0u;
+    r.v[j] &= keep;
+  }
+}
 
 // ---------------------------------------------------------------------------------
 // Per-wave streaming state and tile step.
@@ -834,27 +893,34 @@ __device__ inline void stream_range_from(WaveState<HB>& st, const Pager& pg,
       pg.issue(t, pa, r);
       pa = pb;
       pb = pg.lookup(t + 2);
-      ready_tile(pg, r);
+      ready_tile(pg, r, t);
       compute_tile<Elem, HB>(st, r, qf, t, lim, lane, qk);
     }
   } else {
     // One wave per SIMD, half the waves of a CU at one block: each wave keeps two tiles
     // in flight, so the CU holds as many bytes in flight as there.  Loads of tile t1 (one
-    // past the range) cover no valid rows and read nothing.
+    // past the range) cover no valid rows and read nothing.  The loop has one exit, taken
+    // with only `ra` in flight: with a second exit between the tiles the compiler merged
+    // the two into one block where `rb` may still be in flight, and waited before every
+    // issue of `rb` until 5 to 13 of the 16 loads of `ra` had landed.
     if (t0 >= t1) return;
     typename Pager::Raw ra, rb;
     pg.issue(t0, pa, ra);
-    for (int t = t0;; t += 2) {
+    int t = t0;
+    for (; t + 1 < t1; t += 2) {
       pg.issue(t + 1, pb, rb);
       pa = pg.lookup(t + 2);
-      ready_tile(pg, ra);
+      ready_tile(pg, ra, t);
       compute_tile<Elem, HB>(st, ra, qf, t, lim, lane, qk);
-      if (t + 1 >= t1) break;
       pg.issue(t + 2, pa, ra);
       pb = pg.lookup(t + 3);
-      ready_tile(pg, rb);
+      ready_tile(pg, rb, t + 1);
       compute_tile<Elem, HB>(st, rb, qf, t + 1, lim, lane, qk);
-      if (t + 2 >= t1) break;
+    }
+    if (t < t1) {
+      last_tile(pg);
+      ready_tile(pg, ra, t);
+      compute_tile<Elem, HB>(st, ra, qf, t, lim, lane, qk);
     }
   }
 }
@@ -863,7 +929,9 @@ template <class Elem, int HB, class Pager, int DEPTH = HB>
 __device__ inline void stream_range(WaveState<HB>& st, const Pager& pg, const u32x4 (&qf)[HB][4],
                                     int t0, int t1, int lim, int lane, float qk) {
   if (t0 >= t1) return;
-  stream_range_from<Elem, HB, Pager, DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, pg.lookup(t0),
+  if constexpr (std::is_same_v<Pager, GenericPager>) pg.begin(t0);
+  const typename Pager::Pages first = pg.lookup(t0);
+  stream_range_from<Elem, HB, Pager, DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, first,
                                             pg.lookup(t0 + 1));
 }
 
