@@ -383,18 +383,17 @@ struct AppendPager : FastPager {
     return (unsigned)page < (unsigned)a.num_pages ? rel : -1;
   }
 
-  // Takes the new token's V row (and, with K_REGS, its K row) from v_new / k_new into the
-  // tile's registers and writes both rows into the pools.  Lane (c, g) holds K row c of
-  // each block at bytes 64kk + 16g, and V row 4g + jj of block slot jj at bytes 16c
-  // (FastPager's koff / voff).  The lanes that hold the token reload those registers; the
-  // loads return in issue order, after the pool loads of the same registers.
-  template <bool K_REGS>
+  // Takes the new token's K and V rows from k_new / v_new into the tile's registers and
+  // writes both rows into the pools.  Lane (c, g) holds K row c of each block at bytes 64kk
+  // + 16g, and V row 4g + jj of block slot jj at bytes 16c (FastPager's koff / voff).  The
+  // lanes that hold the token reload those registers; the loads return in issue order,
+  // after the pool loads of the same registers.
   __device__ inline void take_new(int rel, const Pages& p, TileRegs& r) const {
     const int b = rel >> 4, prow = rel & 15;
     const int c = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int bb = 0; bb < 2; ++bb) {
-      if (K_REGS && bb == b && c == prow) {
+      if (bb == b && c == prow) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) r.k[bb][kk] = *(const u32x4*)(kn + kk * 64 + g * 16);
       }
@@ -402,7 +401,10 @@ struct AppendPager : FastPager {
       for (int jj = 0; jj < 4; ++jj)
         if (bb == b && 4 * g + jj == prow) r.v[bb * 4 + jj] = *(const u32x4*)(vn + c * 16);
     }
-    const int page = b ? p.page[1] : p.page[0];
+    write_new(rel, p);
+  }
+  __device__ inline void write_new(int rel, const Pages& p) const {
+    const int page = (rel >> 4) ? p.page[1] : p.page[0];
     int logical, in_page;
     page_of(a, pos, logical, in_page);
     const long dst = (long)page * page_bytes + head_bytes + (long)in_page * (kD * 2) + lane * 4;
@@ -413,7 +415,7 @@ struct AppendPager : FastPager {
   __device__ inline void issue(int tile, const Pages& p, TileRegs& r) const {
     FastPager::issue(tile, p, r);
     const int rel = new_row(tile, p);
-    if (rel >= 0) take_new<true>(rel, p, r);
+    if (rel >= 0) take_new(rel, p, r);
   }
 };
 
@@ -466,13 +468,18 @@ struct ContigPager {
   }
 };
 
-// A 2-byte pager (FastPager, ContigPager, AppendPager) whose K loads take whole 128-byte
-// lines and go straight to LDS, for launches of few units, where what one CU streams
-// bounds the launch: a lone CU streams 35-37 GB/s with the K-operand shape (16 rows x
-// 64 B per instruction) and 45-56 GB/s with whole lines.  K bypasses the registers
-// (buffer_load_dwordx4 ... lds: lane i of an instruction writes the 16 bytes at slab
-// offset 16 i), so a wave keeps two tiles in flight with one tile's V registers more;
-// V is loaded as by the base pager.
+// A 2-byte pager (FastPager, ContigPager, AppendPager) for launches of few units, whose CUs
+// are shared out by output dims: 8 / NV workgroups ("slices") take one unit, each the whole
+// QK product and 16 NV of the 128 output dims, so they need no memory to meet in and a
+// launch without a workspace still uses several CUs per unit.  What one CU streams bounds
+// such a launch (35-37 GB/s with the K-operand shape, 16 rows x 64 B per instruction, 45-56
+// GB/s with whole lines), so
+//   - K takes whole 128-byte lines straight to LDS (buffer_load_dwordx4 ... lds: lane i of
+//     an instruction writes the 16 bytes at slab offset 16 i): it costs no registers, and a
+//     wave keeps two tiles in flight;
+//   - each slice reads only its dims of V (2 NV bytes per lane and token row);
+//   - the slices of a unit run on one XCD in step, so that K, read by each of them, comes
+//     from HBM once (K keeps the default cache policy; each V byte is read by one slice).
 // A slab holds a tile's two 16-token blocks, 16 rows x 256 B each, with
 // 16-byte column `col` of row `row` at position col ^ row: instruction j of a block
 // writes rows 4j .. 4j + 3 (lane (c, g): row 4j + g, position c, so it loads column
@@ -481,33 +488,65 @@ struct ContigPager {
 // lanes.  tile_k of a LineTile reads the MFMA operands back one k-block at a time.
 constexpr int kSlabBytes = 8192;  // one tile's two blocks of K rows
 
-struct LineTile : TileRegs {  // k[][] unused: K is in the slab
+// This lane's NV dims of a V row.
+template <int NV> struct DimsOf;
+template <> struct DimsOf<8> {
+  using Type = u32x4;
+  __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kKvLoadPolicy);
+  }
+  __device__ static inline uint32_t word(const Type& v, int i) { return v[i]; }
+};
+template <> struct DimsOf<4> {
+  using Type = u32x2;
+  __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kKvLoadPolicy);
+  }
+  __device__ static inline uint32_t word(const Type& v, int i) { return v[i]; }
+};
+template <> struct DimsOf<2> {
+  using Type = uint32_t;
+  __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kKvLoadPolicy);
+  }
+  __device__ static inline uint32_t word(const Type& v, int) { return v; }
+};
+
+template <int NV>
+struct LineTile {
+  typename DimsOf<NV>::Type v[8];  // V row of token slot j, this lane's dims
   const uint8_t* rd;  // this lane's K-operand row in the slab: slab + 256 c
   int col;            // g ^ c: k-block kk's 16-byte column is 4 kk ^ col
   int new_row;        // appending pagers: the new token's row of the tile, or -1
   u32x4 k_new;        // ... and bytes 16 c .. +16 of its K row
 };
 
-template <class Base, int SLABS = 1>
+template <class Base, int NV>
 struct Lines : Base {
-  using Raw = LineTile;
-  uint8_t* slab;      // this wave's SLABS x 8 KB of LDS (wave-uniform); tile t uses slab t % SLABS
+  using Raw = LineTile<NV>;
+  uint8_t* slab;      // this wave's two 8 KB slabs of LDS (wave-uniform); tile t uses slab t % 2
   uint32_t kline[4];  // per-lane byte offsets inside a block of instruction j's K row
-  int lane;
+  uint32_t vline[4];  // ... and of V token slot j's dims
+  int lane, slice;
 
-  __device__ Lines(const DecodeArgs& args, int row, int kvh, int limit, int lane_, uint8_t* s)
-      : Base(args, row, kvh, limit, lane_), slab(s), lane(lane_) {
+  __device__ Lines(const DecodeArgs& args, int row, int kvh, int limit, int lane_, uint8_t* s, int slice_)
+      : Base(args, row, kvh, limit, lane_), slab(s), lane(lane_), slice(slice_) {
     const int c = lane_ & 15, g = lane_ >> 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) kline[j] = (4 * j + g) * 256 + (c ^ (4 * j + g)) * 16;
+    for (int j = 0; j < 4; ++j) {
+      kline[j] = (4 * j + g) * 256 + (c ^ (4 * j + g)) * 16;
+      vline[j] = (4 * g + j) * 256 + dim0() * 2;
+    }
   }
+  // This lane's first output dim.
+  __device__ inline int dim0() const { return slice * 16 * NV + (lane & 15) * NV; }
 
   // Rows past the block's valid ones are outside the descriptor and load as 0; their
   // scores are masked in compute_tile whatever the slab holds.  With AppendPager the new
-  // token's V row is taken into the registers here and its K row is loaded beside the
+  // token's V dims are taken into the registers here and its K row is loaded beside the
   // tile, to be put into the slab once the tile has landed there (ready_tile).
-  __device__ inline void issue(int tile, const typename Base::Pages& p, LineTile& r) const {
-    uint8_t* sb = slab + (SLABS == 2 ? (tile & 1) * kSlabBytes : 0);
+  __device__ inline void issue(int tile, const typename Base::Pages& p, Raw& r) const {
+    uint8_t* sb = slab + (tile & 1) * kSlabBytes;
     __amdgpu_buffer_rsrc_t rk[2], rv[2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) this->block_rsrc(tile, b, p, rk[b], rv[b]);
@@ -520,19 +559,22 @@ struct Lines : Base {
       for (int j = 0; j < 4; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rk[b], (__attribute__((address_space(3))) void*)(sb + b * 4096 + j * 1024), 16, kline[j],
-            0, 0, kKvLoadPolicy);
+            0, 0, NV < 8 ? 0 : kKvLoadPolicy);
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        r.v[b * 4 + j] = __builtin_amdgcn_raw_buffer_load_b128(rv[b], this->voff[b * 4 + j], 0, kKvLoadPolicy);
+      for (int j = 0; j < 4; ++j) r.v[b * 4 + j] = DimsOf<NV>::load(rv[b], vline[j]);
     r.new_row = -1;
     if constexpr (std::is_same_v<Base, AppendPager>) {
       r.new_row = this->new_row(tile, p);
       if (r.new_row >= 0) {
         r.k_new = *(const u32x4*)(this->kn + (lane & 15) * 16);
-        this->template take_new<false>(r.new_row, p, r);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (v_slot_token(lane >> 4, j) == r.new_row)
+            r.v[j] = *(const typename DimsOf<NV>::Type*)(this->vn + dim0() * 2);
+        if (slice == 0) this->write_new(r.new_row, p);  // one slice writes the pools
       }
     }
     r.rd = sb + (lane & 15) * 256;
@@ -547,8 +589,8 @@ __device__ inline void ready_tile(const Pager&, Raw&, int) {}
 // The last tile of a range is computed with no further tile's loads behind it.
 template <class Pager>
 __device__ inline void last_tile(const Pager&) {}
-template <class Base, int SLABS>
-__device__ inline void last_tile(const Lines<Base, SLABS>&) {
+template <class Base, int NV>
+__device__ inline void last_tile(const Lines<Base, NV>&) {
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // K in the slab; 8 V loads may remain
 }
 
@@ -559,11 +601,10 @@ __device__ inline void last_tile(const Lines<Base, SLABS>&) {
 // where they are first used, after the scores.  The wait is also a compiler memory
 // barrier, so the slab's reads stay below it; consumed by the tile's MFMAs, they are
 // done before the slab's next loads are issued.
-template <class Base, int SLABS>
-__device__ inline void ready_tile(const Lines<Base, SLABS>& pg, LineTile& r, int) {
+template <class Base, int NV>
+__device__ inline void ready_tile(const Lines<Base, NV>& pg, LineTile<NV>& r, int) {
   const int c = pg.lane & 15, g = pg.lane >> 4;
-  if constexpr (SLABS == 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
   if (r.new_row >= 0) {  // the appended token's K row replaces what the pool held
     const int row = r.new_row & 15;
     if (g == 0) *(u32x4*)(r.rd - c * 256 + (r.new_row >> 4) * 4096 + row * 256 + (c ^ row) * 16) = r.k_new;
@@ -750,9 +791,10 @@ __device__ inline void ready_tile(const GenericPager& pg, TileRegs& r, int tile)
 // ---------------------------------------------------------------------------------
 constexpr float kSlack = 8.0f;
 
-template <int HB>
+// NV: output dims per lane (8, or the fewer of a slice of the dims, see Lines).
+template <int HB, int NV = 8>
 struct WaveState {
-  f32x4 o[HB][8];  // o[hb][jj][i] = O[head hb*16 + 4g + i][dim 8c + jj], relative to m
+  f32x4 o[HB][NV];  // o[hb][jj][i] = O[head hb*16 + 4g + i][dim NV c + jj], relative to m
   float m[HB];     // reference max (log2 units) of head hb*16 + c, uniform over its lanes
   float mx[HB];    // lane-local true running max (log2 units)
   float l[HB];     // lane-partial sum of exp2(x - m)
@@ -767,8 +809,8 @@ __device__ inline u32x4 tile_k(const Fp8Tile& r, int b, int kk) {
   const u32x4 w = r.k[b][kk >> 1];
   return Elem::unpack8((kk & 1) ? u32x2{w[2], w[3]} : u32x2{w[0], w[1]});
 }
-template <class Elem>
-__device__ inline u32x4 tile_k(const LineTile& r, int b, int kk) {
+template <class Elem, int NV>
+__device__ inline u32x4 tile_k(const LineTile<NV>& r, int b, int kk) {
   return *(const u32x4*)(r.rd + b * 4096 + ((4 * kk) ^ r.col) * 16);
 }
 
@@ -788,6 +830,16 @@ __device__ inline void transpose_v(const TileRegs& r, u32x4 (&vt)[8]) {
                                         (jj & 1) ? 0x07060302u : 0x05040100u);
   }
 }
+template <class Elem, int NV>
+__device__ inline void transpose_v(const LineTile<NV>& r, u32x4 (&vt)[NV]) {
+#pragma unroll
+  for (int jj = 0; jj < NV; ++jj)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      vt[jj][q] = __builtin_amdgcn_perm(DimsOf<NV>::word(r.v[2 * q + 1], jj >> 1),
+                                        DimsOf<NV>::word(r.v[2 * q], jj >> 1),
+                                        (jj & 1) ? 0x07060302u : 0x05040100u);
+}
 // fp8 V: the bytes are interleaved first, t = (slot 2q dim 2m, slot 2q + 1 dim 2m, slot 2q
 // dim 2m + 1, slot 2q + 1 dim 2m + 1) with dim counted from 8c, so that the conversion of
 // t's low and high byte pairs yields vt[2m][q] and vt[2m + 1][q].
@@ -805,12 +857,12 @@ __device__ inline void transpose_v(const Fp8Tile& r, u32x4 (&vt)[8]) {
   }
 }
 
-template <class Elem, int HB, class Tile>
-__device__ inline void compute_tile(WaveState<HB>& st, const Tile& r,
+template <class Elem, int HB, int NV, class Tile>
+__device__ inline void compute_tile(WaveState<HB, NV>& st, const Tile& r,
                                     const u32x4 (&qf)[HB][4], int tile, int lim, int lane,
                                     float qk) {
   const int g = lane >> 4;
-  u32x4 vt[8];  // transposed V (before the first PV product)
+  u32x4 vt[NV];  // transposed V (before the first PV product)
   const int tok_base = tile * kTile + 4 * g;
   const bool partial = (tile + 1) * kTile > lim;  // wave-uniform
 #pragma unroll
@@ -847,7 +899,7 @@ __device__ inline void compute_tile(WaveState<HB>& st, const Tile& r,
       for (int i = 0; i < 4; ++i) {
         const float ci = __shfl(corr, 4 * g + i);  // lane 4g + i holds head 4g + i
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) st.o[hb][jj][i] *= ci;
+        for (int jj = 0; jj < NV; ++jj) st.o[hb][jj][i] *= ci;
       }
     }
     float p[8], psum = 0.f;
@@ -870,7 +922,7 @@ __device__ inline void compute_tile(WaveState<HB>& st, const Tile& r,
                               p[2 * q + 1] - __builtin_bit_cast(float, pa[q] & 0xffff0000u));
       }
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) st.o[hb][jj] = Elem::mma(pa, vt[jj], st.o[hb][jj]);
+      for (int jj = 0; jj < NV; ++jj) st.o[hb][jj] = Elem::mma(pa, vt[jj], st.o[hb][jj]);
     }
   }
 }
@@ -882,8 +934,8 @@ __device__ inline void compute_tile(WaveState<HB>& st, const Tile& r,
 // flight per wave on top of that made the work-queue step about 7 % slower).  DEPTH 2:
 // one wave per SIMD keeps the same bytes in flight (the two-head-block kernel and the
 // balanced work-queue schedule).
-template <class Elem, int HB, class Pager, int DEPTH = HB>
-__device__ inline void stream_range_from(WaveState<HB>& st, const Pager& pg,
+template <class Elem, int HB, class Pager, int DEPTH = HB, int NV = 8>
+__device__ inline void stream_range_from(WaveState<HB, NV>& st, const Pager& pg,
                                          const u32x4 (&qf)[HB][4], int t0, int t1, int lim,
                                          int lane, float qk, typename Pager::Pages pa,
                                          typename Pager::Pages pb) {
@@ -925,8 +977,8 @@ __device__ inline void stream_range_from(WaveState<HB>& st, const Pager& pg,
   }
 }
 
-template <class Elem, int HB, class Pager, int DEPTH = HB>
-__device__ inline void stream_range(WaveState<HB>& st, const Pager& pg, const u32x4 (&qf)[HB][4],
+template <class Elem, int HB, class Pager, int DEPTH = HB, int NV = 8>
+__device__ inline void stream_range(WaveState<HB, NV>& st, const Pager& pg, const u32x4 (&qf)[HB][4],
                                     int t0, int t1, int lim, int lane, float qk) {
   if (t0 >= t1) return;
   if constexpr (std::is_same_v<Pager, GenericPager>) pg.begin(t0);
@@ -1412,15 +1464,15 @@ __device__ inline void load_q(const DecodeArgs& a, int q_loaded, int row, int qh
   }
 }
 
-template <int HB>
-__device__ inline void init_state(WaveState<HB>& st) {
+template <int HB, int NV>
+__device__ inline void init_state(WaveState<HB, NV>& st) {
 #pragma unroll
   for (int hb = 0; hb < HB; ++hb) {
     st.m[hb] = -FLT_MAX;
     st.mx[hb] = -FLT_MAX;
     st.l[hb] = 0.f;
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) st.o[hb][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < NV; ++jj) st.o[hb][jj] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 }
 
@@ -1433,19 +1485,20 @@ enum : int { kPgGeneric = 0, kPgFast = 1, kPgContig = 2, kPgFp8 = 3, kPgAppend =
 
 // Streams tiles [t0, t1) of (row, kvh) into the wave state without finishing it, so that
 // several ranges can be streamed into one state (finish_state ends it).  `slab` is the
-// wave's 8 KB of LDS for the whole-line pagers.
-template <class Elem, int HB, int PG, int DEPTH = HB>
-__device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB>& st, const u32x4 (&qf)[HB][4],
+// wave's 16 KB of LDS for the whole-line pagers and `slice` its slice of the output dims.
+template <class Elem, int HB, int PG, int DEPTH = HB, int NV = 8>
+__device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB, NV>& st, const u32x4 (&qf)[HB][4],
                                     int row, int kvh, int t0, int t1, int len, int lane,
                                     bool have_first = false, FastPager::Pages f0 = {},
-                                    FastPager::Pages f1 = {}, uint8_t* slab = nullptr) {
+                                    FastPager::Pages f1 = {}, uint8_t* slab = nullptr, int slice = 0) {
   const long lim_l = (long)t1 * kTile;
   const int lim = uniform(lim_l < len ? (int)lim_l : len);
   const float qk = a.score_scale;
   if constexpr (PG == kPgLines || PG == kPgContigLines || PG == kPgAppendLines) {
     using Base = std::conditional_t<PG == kPgLines, FastPager,
                                     std::conditional_t<PG == kPgContigLines, ContigPager, AppendPager>>;
-    Lines<Base, DEPTH> pg(a, row, kvh, lim, lane, slab);
+    static_assert(DEPTH == 2, "two slabs per wave");
+    Lines<Base, NV> pg(a, row, kvh, lim, lane, slab, slice);
     stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
     // The loop's last loads (the tile after the range, which reads nothing) still write
     // the slab; they are done before the LDS is used for the combine or the workgroup ends.
@@ -1473,8 +1526,8 @@ __device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB>& st, cons
 
 // Ends a wave state: the lane-partial sums and maxima of each head are reduced over the
 // head's four lanes.
-template <int HB>
-__device__ inline void finish_state(WaveState<HB>& st) {
+template <int HB, int NV>
+__device__ inline void finish_state(WaveState<HB, NV>& st) {
 #pragma unroll
   for (int hb = 0; hb < HB; ++hb) {
     st.l[hb] = head_sum(st.l[hb]);
@@ -1482,14 +1535,14 @@ __device__ inline void finish_state(WaveState<HB>& st) {
   }
 }
 
-template <class Elem, int HB, int PG, int DEPTH = HB>
-__device__ inline void stream_unit(const DecodeArgs& a, WaveState<HB>& st, const u32x4 (&qf)[HB][4],
+template <class Elem, int HB, int PG, int DEPTH = HB, int NV = 8>
+__device__ inline void stream_unit(const DecodeArgs& a, WaveState<HB, NV>& st, const u32x4 (&qf)[HB][4],
                                    int row, int kvh, int t0, int t1, int len, int lane,
                                    bool have_first = false, FastPager::Pages f0 = {},
-                                   FastPager::Pages f1 = {}, uint8_t* slab = nullptr) {
+                                   FastPager::Pages f1 = {}, uint8_t* slab = nullptr, int slice = 0) {
   stream_tiles<Elem, HB, PG, DEPTH>(a, st, qf, row, kvh, t0, t1, len, lane, have_first, f0, f1,
-                                    slab);
-  finish_state<HB>(st);
+                                    slab, slice);
+  finish_state(st);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1508,9 +1561,9 @@ struct Dest {
 // One wave's state is the unit's whole state: write it from registers.  Lanes (*, c) hold
 // the softmax state of head hb*16 + c; lane (g, c) holds O of heads hb*16 + 4g + i, dims
 // 8c .. 8c + 7.
-template <class Elem, int HB, bool DIRECT>
-__device__ inline void write_wave_state(const DecodeArgs& a, const WaveState<HB>& st, int qh0,
-                                        int out_row, const Dest& d, int lane) {
+template <class Elem, int HB, bool DIRECT, int NV>
+__device__ inline void write_wave_state(const DecodeArgs& a, const WaveState<HB, NV>& st, int qh0,
+                                        int out_row, const Dest& d, int lane, int slice = 0) {
   const int G = a.group, c = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int hb = 0; hb < HB; ++hb) {
@@ -1518,7 +1571,7 @@ __device__ inline void write_wave_state(const DecodeArgs& a, const WaveState<HB>
     // acc = sum exp(s - m) v; cuh:620-632); the direct op normalises instead.
     const float rescale = __builtin_amdgcn_exp2f(st.m[hb] - st.mx[hb]);
     const float inv_l = st.l[hb] > 0.f ? 1.f / st.l[hb] : 0.f;
-    if (!DIRECT && g == 0 && hb * 16 + c < G) {
+    if (!DIRECT && slice == 0 && g == 0 && hb * 16 + c < G) {
       const long s = d.state0 + (long)(hb * 16 + c) * d.stride;
       put_f32(d.m + s, st.mx[hb] * kLn2, d.coherent);
       put_f32(d.l + s, st.l[hb] * rescale, d.coherent);
@@ -1527,19 +1580,31 @@ __device__ inline void write_wave_state(const DecodeArgs& a, const WaveState<HB>
     for (int i = 0; i < 4; ++i) {
       const int h = hb * 16 + 4 * g + i;  // lane 4g + i holds the state of head h
       const float r = __shfl(DIRECT ? inv_l : rescale, 4 * g + i) * a.v_scale;
-      const f32x4 lo = f32x4{st.o[hb][0][i], st.o[hb][1][i], st.o[hb][2][i], st.o[hb][3][i]} * r;
-      const f32x4 hi = f32x4{st.o[hb][4][i], st.o[hb][5][i], st.o[hb][6][i], st.o[hb][7][i]} * r;
+      float x[NV];
+#pragma unroll
+      for (int jj = 0; jj < NV; ++jj) x[jj] = st.o[hb][jj][i] * r;
       if (h >= G) continue;
+      const int dim = slice * 16 * NV + NV * c;
       if (DIRECT) {
         if (out_row >= 0 && out_row < a.out_rows) {
-          const long e = ((long)out_row * a.hq + qh0 + h) * kD + 8 * c;
-          store_out4<Elem>(a.out, e, lo);
-          store_out4<Elem>(a.out, e + 4, hi);
+          const long e = ((long)out_row * a.hq + qh0 + h) * kD + dim;
+          if constexpr (NV == 2) {
+            *(uint32_t*)(a.out + e * 2) = Elem::pack2(x[0], x[1]);
+          } else {
+#pragma unroll
+            for (int jj = 0; jj < NV; jj += 4)
+              store_out4<Elem>(a.out, e + jj, f32x4{x[jj], x[jj + 1], x[jj + 2], x[jj + 3]});
+          }
         }
       } else {
-        float* dst = d.acc + (d.state0 + (long)h * d.stride) * kD + 8 * c;
-        put_f32x4(dst, lo, d.coherent);
-        put_f32x4(dst + 4, hi, d.coherent);
+        float* dst = d.acc + (d.state0 + (long)h * d.stride) * kD + dim;
+        if constexpr (NV == 2) {
+          *(f32x2*)dst = f32x2{x[0], x[1]};  // no fused merge with slices
+        } else {
+#pragma unroll
+          for (int jj = 0; jj < NV; jj += 4)
+            put_f32x4(dst + jj, f32x4{x[jj], x[jj + 1], x[jj + 2], x[jj + 3]}, d.coherent);
+        }
       }
     }
   }
@@ -1550,12 +1615,13 @@ __device__ inline void write_wave_state(const DecodeArgs& a, const WaveState<HB>
 // result.  LDS: m[w][32] (reference max), l[w][32], x[w][32] (true max),
 // o[w][gh][128] with gh = min(G, chunk).  Starts with a barrier, so LDS can be reused by
 // consecutive units of one workgroup.
-template <class Elem, int HB, int NW, bool DIRECT>
-__device__ inline void combine_waves(const DecodeArgs& a, const WaveState<HB>& st, float* lds,
+template <class Elem, int HB, int NW, bool DIRECT, int NV>
+__device__ inline void combine_waves(const DecodeArgs& a, const WaveState<HB, NV>& st, float* lds,
                                      int qh0, int out_row, const Dest& d, int tid, int lane,
-                                     int wave) {
+                                     int wave, int slice = 0) {
   constexpr int kThreads = NW * 64;
-  constexpr int kChunk = NW == 8 ? 8 : 16;
+  constexpr int kDims = 16 * NV;  // output dims of the workgroup
+  constexpr int kChunk = NW >= 8 ? 8 : 16;
   const int G = a.group, c = lane & 15, g = lane >> 4;
   const int gh = G < kChunk ? G : kChunk;
   float* sm_m = lds;
@@ -1586,14 +1652,20 @@ __device__ inline void combine_waves(const DecodeArgs& a, const WaveState<HB>& s
       for (int i = 0; i < 4; ++i) {
         const int hh = 4 * g + i - sub * kChunk;
         if (hh >= 0 && hh < nh) {
-          float* dst = sm_o + ((long)wave * gh + hh) * kD + 8 * c;
-          *(f32x4*)dst = f32x4{st.o[hb][0][i], st.o[hb][1][i], st.o[hb][2][i], st.o[hb][3][i]};
-          *(f32x4*)(dst + 4) = f32x4{st.o[hb][4][i], st.o[hb][5][i], st.o[hb][6][i], st.o[hb][7][i]};
+          float* dst = sm_o + ((long)wave * gh + hh) * kDims + NV * c;
+          if constexpr (NV == 2) {
+            *(f32x2*)dst = f32x2{st.o[hb][0][i], st.o[hb][1][i]};
+          } else {
+#pragma unroll
+            for (int jj = 0; jj < NV; jj += 4)
+              *(f32x4*)(dst + jj) =
+                  f32x4{st.o[hb][jj][i], st.o[hb][jj + 1][i], st.o[hb][jj + 2][i], st.o[hb][jj + 3][i]};
+          }
         }
       }
       __syncthreads();
-      for (int idx = tid; idx < nh * (kD / 4); idx += kThreads) {
-        const int hh = idx / (kD / 4), dd = (idx % (kD / 4)) * 4;
+      for (int idx = tid; idx < nh * (kDims / 4); idx += kThreads) {
+        const int hh = idx / (kDims / 4), dd = (idx % (kDims / 4)) * 4;
         const int h = h0 + hh;
         float M = -FLT_MAX;
 #pragma unroll
@@ -1604,12 +1676,12 @@ __device__ inline void combine_waves(const DecodeArgs& a, const WaveState<HB>& s
         for (int w = 0; w < NW; ++w) {
           const float e = __builtin_amdgcn_exp2f(sm_m[w * 32 + h] - M);
           L += e * sm_l[w * 32 + h];
-          A += e * *(const f32x4*)(sm_o + ((long)w * gh + hh) * kD + dd);
+          A += e * *(const f32x4*)(sm_o + ((long)w * gh + hh) * kDims + dd);
         }
         if (DIRECT) {
           if (out_row >= 0 && out_row < a.out_rows) {
             const float inv = L > 0.f ? 1.f / L : 0.f;
-            store_out4<Elem>(a.out, ((long)out_row * a.hq + qh0 + h) * kD + dd, A * (inv * a.v_scale));
+            store_out4<Elem>(a.out, ((long)out_row * a.hq + qh0 + h) * kD + slice * kDims + dd, A * (inv * a.v_scale));
           }
         } else {
           // Re-express (L, A) relative to the true max so the partial state is
@@ -1619,8 +1691,8 @@ __device__ inline void combine_waves(const DecodeArgs& a, const WaveState<HB>& s
           for (int w = 0; w < NW; ++w) Mx = fmaxf(Mx, sm_x[w * 32 + h]);
           const float rescale = __builtin_amdgcn_exp2f(M - Mx);
           const long s = d.state0 + (long)h * d.stride;
-          put_f32x4(d.acc + s * kD + dd, A * (rescale * a.v_scale), d.coherent);
-          if (dd == 0) {
+          put_f32x4(d.acc + s * kD + slice * kDims + dd, A * (rescale * a.v_scale), d.coherent);
+          if (slice == 0 && dd == 0) {
             put_f32(d.m + s, Mx * kLn2, d.coherent);
             put_f32(d.l + s, L * rescale, d.coherent);
           }
@@ -1717,19 +1789,20 @@ __device__ inline bool combine_async(const DecodeArgs& a, const WaveState<HB>& s
 // ---------------------------------------------------------------------------------
 constexpr int kSoloTiles = 2;
 
-template <class Elem, int HB, int PG, int MODE, int DEPTH = HB, bool FUSED = false>
+template <class Elem, int HB, int PG, int MODE, int DEPTH = HB, bool FUSED = false, int NV = 8>
 __device__ void solo_unit(const DecodeArgs& a, const Unit& u, int q_loaded, int t0, int t1,
                           const Dest& d, int lane, bool have_first, FastPager::Pages f0,
-                          FastPager::Pages f1, bool fused_all, uint8_t* slab = nullptr) {
+                          FastPager::Pages f1, bool fused_all, uint8_t* slab = nullptr,
+                          int slice = 0) {
   const int qh0 = u.kvh * a.group;
   u32x4 qf[HB][4];
   load_q<HB, PG == kPgFp8>(a, q_loaded, u.row, qh0, lane, qf);
-  WaveState<HB> st;
-  init_state<HB>(st);
+  WaveState<HB, NV> st;
+  init_state(st);
   stream_unit<Elem, HB, PG, DEPTH>(a, st, qf, u.row, u.kvh, t0, t1, u.len, lane, have_first, f0,
-                                   f1, slab);
+                                   f1, slab, slice);
   const int out_row = MODE == kDirect ? (a.out_indices ? a.out_indices[u.row] : u.row) : 0;
-  write_wave_state<Elem, HB, MODE == kDirect>(a, st, qh0, out_row, d, lane);
+  write_wave_state<Elem, HB, MODE == kDirect>(a, st, qh0, out_row, d, lane, slice);
   if constexpr (MODE == kQueue && FUSED) arrive<Elem>(a, u, qh0, lane, 0, 1, fused_all);
 }
 
@@ -1756,7 +1829,12 @@ __device__ inline void zero_empty_rows(const DecodeArgs& a, int tid, int threads
   }
 }
 
-template <class Elem, int HB, int PG, int MODE, int NW, bool ASYNC, int DEPTH = HB, bool FUSED = false>
+//
+// NV < 8: the 8 / NV workgroups of a unit each compute 16 NV of its output dims (Lines).
+// Workgroup b runs on XCD b % 8, so unit u's slices are workgroups u / 8 * 8 * slices +
+// slice * 8 + u % 8.
+template <class Elem, int HB, int PG, int MODE, int NW, bool ASYNC, int DEPTH = HB, bool FUSED = false,
+          int NV = 8>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((HB == 1 && DEPTH == 1) ? 2 : 1)))
 void decode_kernel(DecodeArgs a) {
   constexpr int kWaves = NW;
@@ -1771,6 +1849,14 @@ void decode_kernel(DecodeArgs a) {
   const int lane = tid & 63;
   const int wave = uniform(tid >> 6);
   const int G = a.group;
+  constexpr int kSlices = 8 / NV;
+  int unit = blockIdx.x, slice = 0;
+  if constexpr (kSlices > 1) {
+    static_assert(kLines && MODE != kQueue, "slices of the output dims need the whole-line pagers");
+    unit = (int)(blockIdx.x / (8 * kSlices)) * 8 + (int)(blockIdx.x & 7);
+    slice = (int)(blockIdx.x >> 3) % kSlices;
+    if (unit >= a.batch * a.hkv * (MODE == kSplit ? a.num_splits : 1)) return;  // whole workgroup
+  }
   // Fused merge: whether the queue writes every slot (the arrival count and the merge's
   // slot rule follow from it).  Loaded here, waited for at the arrival.
   int so_first = 0, so_last = 0;
@@ -1809,10 +1895,10 @@ void decode_kernel(DecodeArgs a) {
   } else if constexpr (MODE != kQueue) {
     // The row follows from the workgroup index: its query row is requested (vector load,
     // waited for only by the Q loads) before its length (scalar load) is read.
-    const int row = MODE == kDirect ? (int)blockIdx.x / a.hkv : (int)blockIdx.x / (a.hkv * a.num_splits);
+    const int row = MODE == kDirect ? unit / a.hkv : unit / (a.hkv * a.num_splits);
     q_loaded = load_vector_lanes(a.q_indices ? a.q_indices + row : nullptr,
                                  a.batch < 0 ? lane : 0);  // batch >= 0 (checked on the host)
-    u = resolve_unit<MODE>(a, blockIdx.x);
+    u = resolve_unit<MODE>(a, unit);
   } else {
     u = resolve_unit<MODE>(a, blockIdx.x);
     if (a.q_indices && u.valid) q_loaded = a.q_indices[u.row];
@@ -1827,7 +1913,7 @@ void decode_kernel(DecodeArgs a) {
   const Dest d{a.part_m, a.part_l, a.part_acc, state0, state_stride, fused};
 
   if (MODE != kDirect && u.tb >= u.te) {
-    write_neutral(a, state0, state_stride, G, tid, kThreads, fused);
+    if (slice == 0) write_neutral(a, state0, state_stride, G, tid, kThreads, fused);
     // An item without tiles is one of its row's arrivals too (a queue that writes every
     // slot; the builder emits none).
     if constexpr (fused) arrive<Elem>(a, u, qh0, lane, wave, kWaves, fused_all);
@@ -1839,9 +1925,9 @@ void decode_kernel(DecodeArgs a) {
   const int n = u.te - u.tb;
   if (n <= kSoloTiles) {
     if (wave == 0)
-      solo_unit<Elem, HB, PG, MODE, DEPTH, FUSED>(a, u, q_loaded, u.tb, u.te, d, lane,
+      solo_unit<Elem, HB, PG, MODE, DEPTH, FUSED, NV>(a, u, q_loaded, u.tb, u.te, d, lane,
                                            u.tb == first_tile, first0, first1, fused_all,
-                                           (uint8_t*)lds);
+                                           (uint8_t*)lds, slice);
     return;
   }
 
@@ -1851,22 +1937,22 @@ void decode_kernel(DecodeArgs a) {
   }
   u32x4 qf[HB][4];
   load_q<HB, PG == kPgFp8>(a, q_loaded, u.row, qh0, lane, qf);
-  WaveState<HB> st;
-  init_state<HB>(st);
+  WaveState<HB, NV> st;
+  init_state(st);
 
   // Contiguous sub-range of the unit's tiles for this wave.
   const int w0 = uniform(u.tb + (n * wave) / kWaves);
   const int w1 = uniform(u.tb + (n * (wave + 1)) / kWaves);
   stream_unit<Elem, HB, PG, DEPTH>(a, st, qf, u.row, u.kvh, w0, w1, u.len, lane,
                                    w0 == first_tile, first0, first1,
-                                   (uint8_t*)lds + (kLines ? wave * DEPTH * kSlabBytes : 0));
+                                   (uint8_t*)lds + (kLines ? wave * DEPTH * kSlabBytes : 0), slice);
   const int out_row = MODE == kDirect ? (a.out_indices ? a.out_indices[u.row] : u.row) : 0;
   if constexpr (ASYNC) {
     if (!combine_async<Elem, HB, NW, MODE == kDirect>(a, st, lds, &arrivals, qh0, out_row, d, lane, wave))
       return;
     if constexpr (fused) arrive<Elem>(a, u, qh0, lane, 0, 1, fused_all);
   } else {
-    combine_waves<Elem, HB, NW, MODE == kDirect>(a, st, lds, qh0, out_row, d, tid, lane, wave);
+    combine_waves<Elem, HB, NW, MODE == kDirect>(a, st, lds, qh0, out_row, d, tid, lane, wave, slice);
     if constexpr (fused) arrive<Elem>(a, u, qh0, lane, wave, kWaves, fused_all);
   }
 }
@@ -2295,7 +2381,7 @@ void balanced_decode_kernel(DecodeArgs a) {
             u32x4{(uint32_t)v, (uint32_t)(vb - v + 1), (uint32_t)T, (uint32_t)(T >> 32)};
     }
     WaveState<1> st;
-    init_state<1>(st);
+    init_state(st);
     stream_unit<Elem, 1, PG, 2>(a, st, qf, r, kvh, t0, t1, len, lane, true, f0, f1);
     const long group = (long)r * a.hkv + kvh + v;
     const Dest d{a.part_m, a.part_l, a.part_acc, group * G, 1, false};
@@ -2326,7 +2412,7 @@ __device__ void balanced_merge_fallback(const DecodeArgs& a, int row, int kvh, i
   u32x4 qf[1][4];
   load_q<1, PG == kPgFp8>(a, q_loaded, row, kvh * G, lane, qf);
   WaveState<1> st;
-  init_state<1>(st);
+  init_state(st);
   for (long i0 = 0; T > 0 && i0 < a.num_tasks; i0 += 64) {
     const ItemLane it = load_item_lane(a, i0, lane);
     const int s = it.f[2];
@@ -2344,7 +2430,7 @@ __device__ void balanced_merge_fallback(const DecodeArgs& a, int row, int kvh, i
       if (t1 > t0) stream_tiles<Elem, 1, PG, 2>(a, st, qf, row, kvh, t0, t1, len, lane);
     }
   }
-  finish_state<1>(st);
+  finish_state(st);
   const Dest d{nullptr, nullptr, nullptr, 0, 1, false};
   write_wave_state<Elem, 1, true>(a, st, kvh * G, out_row, d, lane);
 }
@@ -2479,7 +2565,7 @@ int log2_exact(int x) {
 // LDS of a decode workgroup: the barrier combine stages O in chunks of heads (8 with 8
 // waves, 16 with 4); the barrier-free combine holds every wave's O at once.
 size_t lds_bytes(int G, int nw, bool async = false) {
-  const int chunk = async ? G : (nw == 8 ? 8 : 16);
+  const int chunk = async ? G : (nw >= 8 ? 8 : 16);
   return (size_t)(3 * nw * 32 + nw * (G < chunk ? G : chunk) * kD) * sizeof(float);
 }
 
@@ -2603,33 +2689,50 @@ hipError_t launch_decode(const DecodeArgs& a, int grid, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Direct and split launches of few, long units (at most half the CUs, at least 16 tiles
-// each: one row's 8 KV heads with no workspace to split into, or a split launch whose
-// workspace holds no sub-splits): each unit is one workgroup on a CU of its own, so the
-// launch runs at what one CU streams, and whole-line K loads (Lines) raise that.  8 waves,
-// each with two tiles in flight (K in two 8 KB LDS slabs, V in registers: 256 KB per CU,
-// 128 KB of LDS, one workgroup per CU).  C1 (8 units of 1 MB): 21.9 us against 30.4 us
-// with the K-operand loads; 12 waves with one tile each 22.5 us, 16 waves 25.0 us (128
-// registers per wave: the Q fragments spill); 9 or 10 waves with two tiles spill 55-143
-// registers.  Units of 8 tiles or fewer are latency-bound and 0.2-0.4 us slower this way
-// (the 8-wave combine and the LDS round trip).  PKV_LINES=0|1 forces the choice (tuning,
-// tests).
-bool use_lines(int mode, int units, int unit_tiles) {
+// Direct and split launches of at most one unit per CU, of at least 16 tiles each, whose
+// longest units end on CUs that stream alone: launches that leave an eighth of the CUs idle
+// or whose rows differ in length.  A lone CU moves ~512 requests (128-byte lines) per us
+// whatever is in flight, so whole-line K loads (Lines), half the requests of the K-operand
+// shape, shorten the end of the launch.
+//   - At most half the CUs in units: the CUs are shared out by output dims, 4 slices of 32
+//     dims per unit up to a quarter of the CUs, else 2 of 64 (a slice's requests are its
+//     unit's K lines and a quarter or half of the V bytes).  8 waves with two tiles in
+//     flight.  One 2k row without a workspace (8 units): 15.3 us with 4 slices, 17.5 with 2,
+//     21.7 undivided; 32 units 22.7 -> 17.7 us, 64 units 23.9 -> 19.5, 128 units 26.8 -> 24.9;
+//     16 split units of an 8k row 13.4 -> 12.8 us, of a 32k row 30.3 -> 28.2.  Starting the
+//     slices of a unit a quarter of its tiles apart, for more K hits in L2: 16.2 us.
+//   - More units: undivided, 3 waves with two tiles in flight.  256 units of 32 rows of
+//     16-1024 tokens 17.7 -> 14.8 us, 192 of 24 rows to 2048 30.5 -> 23.1, 136 equal ones
+//     19.0 -> 14.9, 224 equal ones 38.7 -> 37.1; 4 waves 14.98, 22.9, 15.3 and 36.8, 2 waves
+//     15.1, 24.7, 16.2 and 37.1.  256 equal units keep every CU streaming to the end and are
+//     better off with the K-operand shape (22.5 against 23.0 us), so launches without
+//     per-row lengths, or of one row, take this path only up to 7/8 of the CUs.
+// Units of 8 tiles or fewer are latency-bound and 0.2-0.4 us slower this way (the LDS round
+// trip).  PKV_LINES=0|1 forces the choice (tuning, tests).
+bool use_lines(int mode, int units, int unit_tiles, bool ragged) {
   static const int forced = [] {
     const char* e = getenv("PKV_LINES");
     return e ? (e[0] == '0' ? 0 : 1) : -1;
   }();
   if (mode == kQueue || forced == 0) return false;
-  return forced == 1 || (2 * units <= cu_count() && unit_tiles >= 16);
+  const int cus = cu_count();
+  return forced == 1 || (unit_tiles >= 16 && (8 * units <= 7 * cus || (ragged && units <= cus)));
 }
 
-constexpr int kLineWaves = 8;
+template <class Elem, int PG, int MODE, int NV, int NW>
+void launch_slices(const DecodeArgs& a, int units, hipStream_t stream) {
+  constexpr int kSlices = 8 / NV;
+  const int grid = kSlices == 1 ? units : (units + 7) / 8 * 8 * kSlices;
+  // At least 96 KB of LDS: one workgroup per CU.
+  const size_t lds = std::max<size_t>({(size_t)NW * 2 * kSlabBytes, (size_t)(96 * 1024), lds_bytes(a.group, NW)});
+  decode_kernel<Elem, 1, PG, MODE, NW, false, 2, false, NV><<<dim3(grid), dim3(NW * 64), lds, stream>>>(a);
+}
 
 template <class Elem, int PG, int MODE>
-hipError_t launch_lines(const DecodeArgs& a, int grid, hipStream_t stream) {
-  const size_t lds = std::max<size_t>((size_t)kLineWaves * 2 * kSlabBytes, lds_bytes(a.group, kLineWaves));
-  decode_kernel<Elem, 1, PG, MODE, kLineWaves, false, 2>
-      <<<dim3(grid), dim3(kLineWaves * 64), lds, stream>>>(a);
+hipError_t launch_lines(const DecodeArgs& a, int units, hipStream_t stream) {
+  if (4 * units <= cu_count()) launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
+  else if (2 * units <= cu_count()) launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
+  else launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
   return hipGetLastError();
 }
 
@@ -2639,7 +2742,7 @@ hipError_t launch_layout(const DecodeArgs& a, int grid, hipStream_t stream) {
   if constexpr (HB == 1 && MODE != kQueue) {
     const int row_tiles = (a.context + kTile - 1) / kTile;
     const int unit_tiles = MODE == kSplit ? row_tiles / a.num_splits : row_tiles;
-    if (!a.kv_fp8 && use_lines(MODE, grid, unit_tiles)) {
+    if (!a.kv_fp8 && use_lines(MODE, grid, unit_tiles, a.seq_lens && a.batch > 1)) {
       if (!a.block_table) return launch_lines<Elem, kPgContigLines, MODE>(a, grid, stream);
       if (a.k_new) return launch_lines<Elem, kPgAppendLines, MODE>(a, grid, stream);  // pages % 16 == 0
       if (a.page_size % 16 == 0) return launch_lines<Elem, kPgLines, MODE>(a, grid, stream);
