@@ -155,6 +155,9 @@ struct DecodeArgs {
   // per decode workgroup the result of its part of the queue check (1 = passed).
   int32_t* bal_plan;
   int32_t* bal_flags;
+  // Grid ops: the workgroups form a (splits, Hkv, batch) grid, so that a unit's row, KV head
+  // and split need no division (a (units) grid when a dimension exceeds the grid limits).
+  int32_t unit_grid;
 };
 
 // ---------------------------------------------------------------------------------
@@ -1043,23 +1046,34 @@ __device__ inline Unit resolve_unit(const DecodeArgs& a, int idx) {
   u.slot_base = 0;
   u.row_splits = 1;
   if (MODE == kDirect) {
-    u.row = idx / a.hkv;
-    u.kvh = idx - u.row * a.hkv;
+    u.row = a.unit_grid ? (int)blockIdx.z : idx / a.hkv;
+    u.kvh = a.unit_grid ? (int)blockIdx.y : idx - u.row * a.hkv;
     u.split = 0;
     u.len = row_length(a, u.row);
     u.tb = 0;
     u.te = ceil_tiles(u.len);
   } else if (MODE == kSplit) {
-    const int per_row = a.hkv * a.num_splits;
-    u.row = idx / per_row;
-    const int rem = idx - u.row * per_row;
-    u.kvh = rem / a.num_splits;
-    u.split = rem - u.kvh * a.num_splits;
+    if (a.unit_grid) {
+      u.row = blockIdx.z;
+      u.kvh = blockIdx.y;
+      u.split = blockIdx.x;
+    } else {
+      const int per_row = a.hkv * a.num_splits;
+      u.row = idx / per_row;
+      const int rem = idx - u.row * per_row;
+      u.kvh = rem / a.num_splits;
+      u.split = rem - u.kvh * a.num_splits;
+    }
     u.len = row_length(a, u.row);
     const int total = ceil_tiles(u.len);
-    // Row-local split bounds, cuh:330-337.
-    u.tb = (int)(((long)total * u.split) / a.num_splits);
-    u.te = (int)(((long)total * (u.split + 1)) / a.num_splits);
+    // Row-local split bounds, cuh:330-337 (num_splits <= ceil(context / 32) < 2^26).
+    if (total < 65536 && a.num_splits < 65536) {
+      u.tb = (int)((uint32_t)total * (uint32_t)u.split / (uint32_t)a.num_splits);
+      u.te = (int)((uint32_t)total * (uint32_t)(u.split + 1) / (uint32_t)a.num_splits);
+    } else {
+      u.tb = (int)(((long)total * u.split) / a.num_splits);
+      u.te = (int)(((long)total * (u.split + 1)) / a.num_splits);
+    }
   } else {
     const int32_t* w = a.work_items + (long)idx * 5;
     const int row = load_scalar(w + 0), kvh = load_scalar(w + 1), split = load_scalar(w + 2);
@@ -1096,12 +1110,12 @@ __device__ inline float get_f32(const float* p) {
   if (COHERENT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return *p;
 }
-template <bool COHERENT>
-__device__ inline f32x2 get_f32x2(const float* p) {
-  if (COHERENT)
-    return __builtin_bit_cast(f32x2, __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT));
-  return *(const f32x2*)p;
+__device__ inline f32x4 get_f32x4_coherent(const float* p) {
+  const f32x2 lo = __builtin_bit_cast(f32x2, __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT));
+  const f32x2 hi = __builtin_bit_cast(f32x2, __hip_atomic_load((const uint64_t*)p + 1, __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT));
+  return f32x4{lo[0], lo[1], hi[0], hi[1]};
 }
 // Waits until every memory access this wave issued has completed.
 
@@ -1163,70 +1177,95 @@ __device__ inline float wave_sum(float x) {
 // L = sum e^(m - M) l, A = sum e^(m - M) acc, O = A / L (0 when L == 0).  Slot s's state
 // index is base + s * stride.  In queue mode, slots of splits the builder leaves empty
 // (split0 + s of nsplit splits over `total` tiles) hold no state and are skipped; the
-// reference reads them uninitialised.  All loads of a chunk of up to 32 slots are
-// issued together: lane s loads slot s's (m, l) and each lane its two dims of every
-// slot's acc.  Lane owns output dims 2*lane, 2*lane + 1 of `out` (128 elements).
+// reference reads them uninitialised.  All loads of a chunk of up to 32 slots are issued
+// together: each 16-byte load takes four dims of two slots, the even ones in lanes 0-31 and
+// the odd ones in lanes 32-63.
+//
+// A merge is one wave's chain of instructions behind one or two round trips (~2.6 ns for
+// each instruction of a lone wave), so two states per instruction count, and weights that
+// the multiply reads through DPP: the fold of 32 states is ~130 instructions, ~280 with one
+// state per load and a readlane per weight.  Kernel traces before and after, with the merges'
+// grids free of divisions: 3.4 -> 3.0 us (one 2k row, 32 splits), balanced schedule 5.7 ->
+// 4.6 (8 bimodal rows) and 5.8 -> 4.0 us (fp8).
 // ---------------------------------------------------------------------------------
 constexpr int kMergeChunk = 32;
 
-// Running LSE merge held by one wave; lane owns output dims 2*lane, 2*lane + 1.
+// The state whose (m, l) a lane holds: each row of 16 lanes holds the 16 states of its half
+// (rows 0 and 1 the even ones, rows 2 and 3 the odd ones).
+__device__ inline int fold_state(int lane) { return 2 * (lane & 15) + (lane >> 5); }
+
+// Running LSE merge held by one wave: lane h * 32 + q sums dims 4q .. 4q + 3 of the even (h
+// = 0) or odd (h = 1) states; the two halves are added by total().
 struct LseAcc {
   float M = -FLT_MAX, L = 0.f;
-  f32x2 A = {0.f, 0.f};
+  f32x4 A = {0.f, 0.f, 0.f, 0.f};
 
-  // Folds in up to 32 states: lane j holds (ms, ls) of state j (valid when ok); v[j] holds
-  // this lane's two dims of state j's acc.
-  __device__ inline void fold(bool ok, float ms, float ls, const f32x2 (&v)[kMergeChunk]) {
+  // x of lane I of the lane's row of 16 (row_newbcast:I).
+  template <int I>
+  __device__ static inline float row_lane(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + I,
+                                                                 0xf, 0xf, false));
+  }
+  template <int I>
+  __device__ inline void add_states(float w, const f32x4 (&v)[kMergeChunk / 2], bool select) {
+    if constexpr (I < kMergeChunk / 2) {
+      const float wi = row_lane<I>(w);
+      if (select) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) A[k] += wi != 0.f ? wi * v[I][k] : 0.f;
+      } else {
+        A += wi * v[I];
+      }
+      add_states<I + 1>(w, v, select);
+    }
+  }
+
+  // Folds in up to 32 states: lane j holds (ms, ls) of state fold_state(j) (live when ok);
+  // v[i] holds this lane's dims of state 2i or 2i + 1, 0 past the n states.
+  __device__ inline void fold(bool ok, float ms, float ls, const f32x4 (&v)[kMergeChunk / 2], int n, int lane) {
     const float cm = wave_max(ok ? ms : -FLT_MAX);
     const float m_new = fmaxf(M, cm);
     const float corr = __builtin_amdgcn_exp2f((M - m_new) * kLog2e);
     M = m_new;
     const float w = ok ? __builtin_amdgcn_exp2f((ms - M) * kLog2e) : 0.f;
-    L = L * corr + wave_sum(ok ? w * ls : 0.f);  // select: skipped slots may hold NaN
+    // Each state is held by two rows and counted in one; select: skipped slots may hold NaN.
+    L = L * corr + wave_sum(ok && !(lane & 16) ? w * ls : 0.f);
     A *= corr;
+    // States without weight (skipped slots, or an underflow) add nothing, whatever they hold.
+    if (__builtin_amdgcn_ballot_w64(fold_state(lane) < n && w == 0.f) == 0) add_states<0>(w, v, false);
+    else add_states<0>(w, v, true);
+  }
+
+  // This lane's four dims over all states, in both halves.
+  __device__ inline f32x4 total() const {
+    f32x4 t;
 #pragma unroll
-    for (int j = 0; j < kMergeChunk; ++j) {
-      const float wj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), j));
-      A[0] += wj != 0.f ? wj * v[j][0] : 0.f;  // select, not multiply: skipped slots may hold NaN
-      A[1] += wj != 0.f ? wj * v[j][1] : 0.f;
-    }
+    for (int k = 0; k < 4; ++k) t[k] = A[k] + __shfl_xor(A[k], 32);
+    return t;
   }
 
   template <class Elem>
   __device__ inline void store(uint8_t* out, int lane) const {
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    *(uint32_t*)(out + 4 * lane) = Elem::pack2(A[0] * inv, A[1] * inv);
+    const f32x4 t = total() * inv;
+    if (lane < 32) store_out4<Elem>(out, 4 * lane, t);
   }
 };
 
-// Up to 32 slot states as one wave loads them: lane j holds (m, l) of slot c0 + j and
-// v[j] this lane's two dims of that slot's acc.  All loads are issued together; the acc
-// of slots past the chunk (n, uniform) is not loaded (v[j] = 0, and fold gives those
-// slots weight 0), since a merge of many short rows would otherwise spend most of its
-// time re-reading the last state.
+// Up to 32 slot states as one wave loads them.  All loads are issued together; slots past
+// the chunk (n, uniform) are not loaded (v = 0), since a merge of many short rows would
+// otherwise spend most of its time re-reading the last state.
 struct SlotChunk {
   float ms, ls;
-  f32x2 v[kMergeChunk];
+  f32x4 v[kMergeChunk / 2];
 };
 
-template <bool COHERENT>
-__device__ inline void load_chunk(SlotChunk& c, const float* pm, const float* pl, const float* pacc,
-                                  long base, long stride, int c0, int n, int lane) {
-  n = uniform(n);
-  const int s_lane = c0 + (lane < n ? lane : n - 1);
-  c.ms = get_f32<COHERENT>(pm + base + (long)s_lane * stride);
-  c.ls = get_f32<COHERENT>(pl + base + (long)s_lane * stride);
-#pragma unroll
-  for (int j = 0; j < kMergeChunk; ++j)
-    c.v[j] = j < n ? get_f32x2<COHERENT>(pacc + (base + (long)(c0 + j) * stride) * kD + 2 * lane)
-                   : f32x2{0.f, 0.f};
-}
-
-// load_chunk through buffer descriptors that cover the chunk's states (n >= 1): when
-// `enable` is false they cover nothing, and the loads return zeros without reading memory.
+// Loads slots [c0, c0 + n) through buffer descriptors that cover exactly their states (n >=
+// 1): lanes past them read zeros, and when `enable` is false the descriptors cover nothing.
 __device__ inline void load_chunk_if(SlotChunk& c, const float* pm, const float* pl, const float* pacc,
-                                     long base, long stride, int n, int lane, bool enable) {
+                                     long base, long stride, int c0, int n, int lane, bool enable) {
   n = uniform(n);
+  base += c0 * stride;
   const int span = enable ? (int)((long)(n - 1) * stride + 1) : 0;  // states from base
   const __amdgpu_buffer_rsrc_t rm =
       __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(pm + base), (short)0, uniform(span * 4), kRsrcWord3);
@@ -1234,14 +1273,35 @@ __device__ inline void load_chunk_if(SlotChunk& c, const float* pm, const float*
       __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(pl + base), (short)0, uniform(span * 4), kRsrcWord3);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(pacc + base * kD), (short)0, uniform(span * kD * 4), kRsrcWord3);
-  const int s_lane = lane < n ? lane : n - 1;
+  const int s_lane = fold_state(lane) < n ? fold_state(lane) : n - 1;
   c.ms = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (int)(s_lane * stride * 4), 0, 0));
   c.ls = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, (int)(s_lane * stride * 4), 0, 0));
+  const int pair = (int)(2 * stride) * (kD * 4);
+  const int off = (int)((lane >> 5) * stride) * (kD * 4) + (lane & 31) * 16;
 #pragma unroll
-  for (int j = 0; j < kMergeChunk; ++j)
-    c.v[j] = j < n ? __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(
-                                                   ra, (int)((j * stride * kD + 2 * lane) * 4), 0, 0))
-                   : f32x2{0.f, 0.f};
+  for (int i = 0; i < kMergeChunk / 2; ++i)
+    c.v[i] = 2 * i < n ? __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, off + i * pair, 0, 0))
+                       : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// The same with agent-scope loads, of states written by other workgroups of the launch.
+template <bool COHERENT>
+__device__ inline void load_chunk(SlotChunk& c, const float* pm, const float* pl, const float* pacc,
+                                  long base, long stride, int c0, int n, int lane) {
+  if constexpr (!COHERENT) {
+    load_chunk_if(c, pm, pl, pacc, base, stride, c0, n, lane, true);
+  } else {
+    n = uniform(n);
+    const int s_lane = c0 + (fold_state(lane) < n ? fold_state(lane) : n - 1);
+    c.ms = get_f32<true>(pm + base + (long)s_lane * stride);
+    c.ls = get_f32<true>(pl + base + (long)s_lane * stride);
+#pragma unroll
+    for (int i = 0; i < kMergeChunk / 2; ++i) {
+      const int j = 2 * i + (lane >> 5);
+      c.v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (j < n) c.v[i] = get_f32x4_coherent(pacc + (base + (long)(c0 + j) * stride) * kD + 4 * (lane & 31));
+    }
+  }
 }
 
 // Whether slot s of a row holds a state.  In queue mode the builder leaves splits with no
@@ -1275,8 +1335,9 @@ __device__ inline void fold_slots(LseAcc& acc, const float* pm, const float* pl,
     const int n = count - c0 < kMergeChunk ? count - c0 : kMergeChunk;
     SlotChunk c;
     load_chunk<COHERENT>(c, pm, pl, pacc, base, stride, c0, n, lane);
-    acc.fold(lane < n && slot_live<QUEUE>(c0 + lane, count, total, nsplit, split0, all), c.ms,
-             c.ls, c.v);
+    const int st = fold_state(lane);
+    acc.fold(st < n && slot_live<QUEUE>(c0 + st, count, total, nsplit, split0, all), c.ms, c.ls, c.v, n,
+             lane);
   }
 }
 
@@ -1296,8 +1357,9 @@ __device__ inline void fold_slots_pipelined(LseAcc& acc, const float* pm, const 
     if (c1 < count)
       load_chunk<false>(nxt, pm, pl, pacc, base, stride, c1,
                         count - c1 < kMergeChunk ? count - c1 : kMergeChunk, lane);
-    acc.fold(lane < n && slot_live<QUEUE>(c0 + lane, count, total, nsplit, split0), cur.ms, cur.ls,
-             cur.v);
+    const int st = fold_state(lane);
+    acc.fold(st < n && slot_live<QUEUE>(c0 + st, count, total, nsplit, split0), cur.ms, cur.ls, cur.v, n,
+             lane);
     cur = nxt;
   }
 }
@@ -1306,9 +1368,8 @@ __device__ inline void fold_slots_pipelined(LseAcc& acc, const float* pm, const 
 // flight at once (one memory round trip; a wave tracks at most 63 vector loads, so the
 // 8-byte loads of fold_slots fit 32 states per round trip).  Lanes 0-31 load the even
 // states and lanes 32-63 the odd ones with 16-byte loads (4 dims per lane): 2 states per
-// load.  Lane j holds (m, l) of states j and j + 64.  Each half accumulates its states;
-// the halves are added and the result is returned in the LseAcc layout (lane owns dims
-// 2 lane, 2 lane + 1).  States are base + s * stride, s < n (wave-uniform, 1 <= n <=
+// load.  Lane j holds (m, l) of states j and j + 64.  Each half accumulates its states (the
+// LseAcc layout).  States are base + s * stride, s < n (wave-uniform, 1 <= n <=
 // kWideStates); in queue mode, slots of empty splits are skipped as in fold_slots.
 constexpr int kWideLoads = 56;
 constexpr int kWideStates = 2 * kWideLoads;
@@ -1345,15 +1406,9 @@ __device__ inline void fold_wide(LseAcc& acc, const float* pm, const float* pl, 
 #pragma unroll
     for (int k = 0; k < 4; ++k) A[k] += w != 0.f ? w * v[i][k] : 0.f;  // select: unused slots may hold NaN
   }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) A[k] += __shfl_xor(A[k], 32);
-  // Lane j's dims 2j, 2j + 1 sit in lane j / 2 (components 0-1 or 2-3).
-  const int src = (lane >> 1) & 31;
-  const float x0 = __shfl(A[0], src), x1 = __shfl(A[1], src);
-  const float x2 = __shfl(A[2], src), x3 = __shfl(A[3], src);
   acc.M = M;
   acc.L = L;
-  acc.A = (lane & 1) ? f32x2{x2, x3} : f32x2{x0, x1};
+  acc.A = A;
 }
 
 // Fused merge of query head qh of a work-queue row by one wave, run by the last work item
@@ -1895,7 +1950,8 @@ void decode_kernel(DecodeArgs a) {
   } else if constexpr (MODE != kQueue) {
     // The row follows from the workgroup index: its query row is requested (vector load,
     // waited for only by the Q loads) before its length (scalar load) is read.
-    const int row = MODE == kDirect ? unit / a.hkv : unit / (a.hkv * a.num_splits);
+    const int row = a.unit_grid ? (int)blockIdx.z
+                                : (MODE == kDirect ? unit / a.hkv : unit / (a.hkv * a.num_splits));
     q_loaded = load_vector_lanes(a.q_indices ? a.q_indices + row : nullptr,
                                  a.batch < 0 ? lane : 0);  // batch >= 0 (checked on the host)
     u = resolve_unit<MODE>(a, unit);
@@ -1975,15 +2031,14 @@ struct MergeArgs {
   int32_t total_slots;           // queue mode
   int32_t context, max_tokens;   // split mode length fallback / clamp
   int32_t num_tasks, hkv;        // queue mode: the queue's item count (-1: unknown) and Hkv
+  int32_t head_grid;             // the grid is (Hq, batch), not (batch * Hq)
 };
 
 template <class Elem, bool QUEUE>
 __global__ __launch_bounds__(64) void merge_kernel(MergeArgs a) {
-  const int wave_id = blockIdx.x;  // one wave per workgroup
-  const int lane = threadIdx.x;
-  if (wave_id >= a.batch * a.hq) return;
-  const int row = uniform(wave_id / a.hq);
-  const int qh = uniform(wave_id - row * a.hq);
+  const int lane = threadIdx.x;  // one wave per workgroup
+  const int row = a.head_grid ? (int)blockIdx.y : uniform((int)blockIdx.x / a.hq);
+  const int qh = a.head_grid ? (int)blockIdx.x : uniform((int)blockIdx.x - row * a.hq);
   // The output row is loaded first and waited for last, so it costs no round trip of its own.
   const int out_row_loaded = load_vector_deferred(a.out_indices ? a.out_indices + row : nullptr);
   int count, total = 0, nsplit = 1, split0 = 0;
@@ -2005,7 +2060,7 @@ __global__ __launch_bounds__(64) void merge_kernel(MergeArgs a) {
                                                       uniform(so_last));
     const int per_row = a.total_slots / a.batch;
     const bool guess = per_row > 0 && per_row * a.batch == a.total_slots;
-    load_chunk_if(guessed, a.part_m, a.part_l, a.part_acc, (long)row * per_row * a.hq + qh, a.hq,
+    load_chunk_if(guessed, a.part_m, a.part_l, a.part_acc, (long)row * per_row * a.hq + qh, a.hq, 0,
                   per_row < 1 ? 1 : (per_row < kMergeChunk ? per_row : kMergeChunk), lane, guess);
     hit = guess && o0 == row * per_row && o1 - o0 == per_row;
     const int first = o0 < 0 ? 0 : o0;
@@ -2032,14 +2087,14 @@ __global__ __launch_bounds__(64) void merge_kernel(MergeArgs a) {
     // not branched on, so their loads stay ahead of the wait for the offsets.
     const int n = count < 1 ? 1 : (count < kMergeChunk ? count : kMergeChunk);
     SlotChunk c;
-    if (!hit) load_chunk_if(c, a.part_m, a.part_l, a.part_acc, base, stride, n, lane, count > 0);
+    if (!hit) load_chunk_if(c, a.part_m, a.part_l, a.part_acc, base, stride, 0, n, lane, count > 0);
     c.ms = hit ? guessed.ms : c.ms;
     c.ls = hit ? guessed.ls : c.ls;
 #pragma unroll
-    for (int j = 0; j < kMergeChunk; ++j) c.v[j] = hit ? guessed.v[j] : c.v[j];
-    acc.fold(lane < count && lane < kMergeChunk &&
-                 slot_live<QUEUE>(lane, count, total, nsplit, split0, all),
-             c.ms, c.ls, c.v);
+    for (int i = 0; i < kMergeChunk / 2; ++i) c.v[i] = hit ? guessed.v[i] : c.v[i];
+    const int st = fold_state(lane);
+    acc.fold(st < count && slot_live<QUEUE>(st, count, total, nsplit, split0, all), c.ms, c.ls, c.v, n,
+             lane);
     c_begin = kMergeChunk;
   }
   fold_slots<QUEUE, false>(acc, a.part_m, a.part_l, a.part_acc, base, stride, count, total, nsplit,
@@ -2464,15 +2519,13 @@ template <class Elem, bool WIDE, int PG>
 __global__ __launch_bounds__(kBalMergeWaves * 64) void balanced_merge_kernel(DecodeArgs a, int waves,
                                                                              int check_wgs) {
   __shared__ float sm_ml[kBalMergeWaves][2];
-  __shared__ f32x2 sm_a[kBalMergeWaves][64];
+  __shared__ f32x4 sm_a[kBalMergeWaves][32];
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int nw = uniform(blockDim.x >> 6);
-  const int wg = blockIdx.x;
-  if (wg >= a.batch * a.hq) return;  // whole workgroup
-  const int row = uniform(wg / a.hq);
-  const int qh = uniform(wg - row * a.hq);
-  const int kvh = uniform(qh / a.group), h = qh - kvh * a.group;
+  // (G, Hkv, batch) grid
+  const int row = blockIdx.z, kvh = blockIdx.y, h = blockIdx.x;
+  const int qh = kvh * a.group + h;
   // One round trip: the output row, the row's length and the pair's plan entry (written by
   // the decode's wave that holds the pair's first tile) are loaded together.
   const int out_row_loaded = load_vector_deferred(a.out_indices ? a.out_indices + row : nullptr);
@@ -2510,31 +2563,30 @@ __global__ __launch_bounds__(kBalMergeWaves * 64) void balanced_merge_kernel(Dec
   else
     fold_slots_pipelined<true>(acc, a.part_m, a.part_l, a.part_acc, base + (long)c0 * a.group,
                                a.group, c1 - c0, T, waves, va + c0, lane);
-  float M = acc.M, L = acc.L;
-  f32x2 A = acc.A;
+  float L = acc.L;
+  f32x4 A = acc.total();
   if (nw > 1) {
     if (lane == 0) {
       sm_ml[wave][0] = acc.M;
       sm_ml[wave][1] = acc.L;
     }
-    sm_a[wave][lane] = acc.A;
+    if (lane < 32) sm_a[wave][lane] = A;
     __syncthreads();
     if (wave != 0) return;
-    M = -FLT_MAX;
+    float M = -FLT_MAX;
     for (int w = 0; w < nw; ++w) M = fmaxf(M, sm_ml[w][0]);
     L = 0.f;
-    A = f32x2{0.f, 0.f};
+    A = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int w = 0; w < nw; ++w) {
       const float e = __builtin_amdgcn_exp2f((sm_ml[w][0] - M) * kLog2e);
       L += e * sm_ml[w][1];
-      A += e * sm_a[w][lane];
+      A += e * sm_a[w][lane & 31];
     }
   }
   const int out_row = a.out_indices ? uniform(out_row_loaded) : row;
-  if (out_row < 0 || out_row >= a.out_rows) return;
+  if (out_row < 0 || out_row >= a.out_rows || lane >= 32) return;
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  *(uint32_t*)(a.out + ((long)out_row * a.hq + qh) * kD * 2 + 4 * lane) =
-      Elem::pack2(A[0] * inv, A[1] * inv);
+  store_out4<Elem>(a.out, ((long)out_row * a.hq + qh) * kD + 4 * lane, A * inv);
 }
 
 // ---------------------------------------------------------------------------------
@@ -2649,6 +2701,17 @@ bool use_async_combine(int units) {
   return units >= 3 * cu_count();
 }
 
+// The workgroups of a launch of `units` units, in unit order: (splits, Hkv, batch) for the
+// grid ops.  With one-dimensional units and 64-bit split bounds the divisions of
+// resolve_unit were ~500 scalar instructions at each workgroup's start: one 32k row in 32
+// splits 26.14 against 25.77 us.
+constexpr int kMaxGridYZ = 65535;
+template <int MODE>
+dim3 unit_grid(DecodeArgs& a, int units) {
+  a.unit_grid = MODE != kQueue && a.hkv <= kMaxGridYZ && a.batch <= kMaxGridYZ;
+  return a.unit_grid ? dim3(MODE == kSplit ? a.num_splits : 1, a.hkv, a.batch) : dim3(units);
+}
+
 // A work-queue launch with the fused merge (merge_counters set) runs its own kernel: the
 // arrivals and the in-kernel merge are compiled only into it, so the unfused kernel's
 // tile loop keeps the scalar registers they would take (the queue kernels spilled
@@ -2662,7 +2725,9 @@ void launch_kernel(const DecodeArgs& a, int grid, size_t lds, hipStream_t stream
       return;
     }
   }
-  decode_kernel<Elem, HB, PG, MODE, NW, ASYNC, DEPTH, false><<<dim3(grid), dim3(NW * 64), lds, stream>>>(a);
+  DecodeArgs u = a;
+  const dim3 units = unit_grid<MODE>(u, grid);
+  decode_kernel<Elem, HB, PG, MODE, NW, ASYNC, DEPTH, false><<<units, dim3(NW * 64), lds, stream>>>(u);
 }
 
 template <class Elem, int HB, int PG, int MODE>
@@ -2722,10 +2787,12 @@ bool use_lines(int mode, int units, int unit_tiles, bool ragged) {
 template <class Elem, int PG, int MODE, int NV, int NW>
 void launch_slices(const DecodeArgs& a, int units, hipStream_t stream) {
   constexpr int kSlices = 8 / NV;
-  const int grid = kSlices == 1 ? units : (units + 7) / 8 * 8 * kSlices;
+  DecodeArgs u = a;
+  u.unit_grid = 0;
+  const dim3 grid = kSlices == 1 ? unit_grid<MODE>(u, units) : dim3((units + 7) / 8 * 8 * kSlices);
   // At least 96 KB of LDS: one workgroup per CU.
   const size_t lds = std::max<size_t>({(size_t)NW * 2 * kSlabBytes, (size_t)(96 * 1024), lds_bytes(a.group, NW)});
-  decode_kernel<Elem, 1, PG, MODE, NW, false, 2, false, NV><<<dim3(grid), dim3(NW * 64), lds, stream>>>(a);
+  decode_kernel<Elem, 1, PG, MODE, NW, false, 2, false, NV><<<grid, dim3(NW * 64), lds, stream>>>(u);
 }
 
 template <class Elem, int PG, int MODE>
@@ -2773,9 +2840,10 @@ int dispatch_decode(const DecodeArgs& a, int dtype, int grid, hipStream_t stream
 // One wave per workgroup, so the (row, head) waves spread over all CUs: each wave's
 // ~10 KB of states then shares its CU's load bandwidth with fewer others (measured: C4
 // 49.9 against 50.4 us and C1 10.3 against 10.5 us with four waves per workgroup).
-int dispatch_merge(const MergeArgs& m, bool queue, int dtype, hipStream_t stream) {
-  const int grid = m.batch * m.hq;
-  if (grid == 0) return PKV_OK;
+int dispatch_merge(MergeArgs m, bool queue, int dtype, hipStream_t stream) {
+  if (m.batch * m.hq == 0) return PKV_OK;
+  m.head_grid = m.batch <= kMaxGridYZ;
+  const dim3 grid = m.head_grid ? dim3(m.hq, m.batch) : dim3(m.batch * m.hq);
   if (dtype == PKV_DTYPE_F16) {
     if (queue) merge_kernel<Half, true><<<grid, 64, 0, stream>>>(m);
     else merge_kernel<Half, false><<<grid, 64, 0, stream>>>(m);
@@ -3174,7 +3242,7 @@ int balanced_waves(const Geometry& g, size_t ws_bytes, int fused_merge, bool fp8
   }();
   if (!on || fused_merge || g.hkv <= 0 || g.batch <= 0) return 0;
   const int G = g.hq / g.hkv;
-  if (G > 16 || g.page_size % 16 != 0 || g.batch > 64 * kBalRowChunks) return 0;
+  if (G > 16 || g.page_size % 16 != 0 || g.batch > 64 * kBalRowChunks || g.hkv > kMaxGridYZ) return 0;
   if (balanced_bytes((long)g.batch * g.hkv, (long)kBalWavesMax * cu_count(), G) > ws_bytes) return 0;
   return bal_waves_per_cu(fp8) * cu_count();
 }
@@ -3229,13 +3297,13 @@ int run_workqueue(const QueueCall& c, int32_t fused_merge, hipStream_t stream, c
       if (e != hipSuccess) return fail(PKV_ERR_LAUNCH, "decode launch failed: %s", hipGetErrorString(e));
     }
     if (stages & 2) {
-      const int grid = c.g.batch * c.g.hq;
+      const dim3 grid(a.group, c.g.hkv, c.g.batch);
       // Waves per (row, query head): as many as the decode ran per CU (a pair's pieces
       // scale with them; C4 step 43.0 against 43.4 us with 4 after two decode waves, fp8
       // merge stage 5.9-6.2 against 6.9-7.0 us with 2 after four), at most the number that
       // keeps the grid within ~8 waves per CU.
       int merge_waves = wg_waves;
-      while (merge_waves > 1 && (long)grid * merge_waves > 8L * cu_count()) merge_waves >>= 1;
+      while (merge_waves > 1 && (long)c.g.batch * c.g.hq * merge_waves > 8L * cu_count()) merge_waves >>= 1;
       const int block = merge_waves * 64;
       // The wide fold (one round trip for up to kWideStates groups, ~250 VGPRs) where a
       // merge wave's share can exceed one chunk: few pairs per merge wave.
