@@ -556,8 +556,9 @@ int pkv_paged_attention_workqueue_append(
 
 /* The fp8-K/V ops with the append: k_new / v_new are in `dtype` and stored as
  * pkv_append_kv_fp8 stores them, e4m3(clamp(x / k_scale)) and e4m3(clamp(x / v_scale)).
- * Same result as pkv_append_kv_fp8 followed by the fp8 op, which is what they run (two
- * launches; an in-decode fp8 append measured slower).  v_scale must be positive. */
+ * Same result as pkv_append_kv_fp8 followed by the fp8 op, which is what they run but for
+ * the work-queue op's balanced schedule, whose decode writes the tokens itself (no two rows
+ * may share a tail page, as above).  v_scale must be positive. */
 int pkv_paged_attention_indexed_fp8_append(
     const void* q_source, int32_t q_rows,
     const void* k_pages, const void* v_pages,

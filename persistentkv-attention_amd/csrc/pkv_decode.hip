@@ -39,6 +39,7 @@
 #include <vector>
 
 #include "pkv.h"
+#include "pkv_e4m3.h"
 
 namespace pkv {
 
@@ -146,8 +147,10 @@ struct DecodeArgs {
   // Contiguous layout only: unit kv head v reads the K/V of head v / kv_div (1, or G for
   // the query-head baseline, whose units are single query heads).
   int32_t kv_div;
-  // Fused append (paged fp16 / bf16, pages a multiple of 16), else null: each row's
-  // newest token, [B, Hkv, 128] in the KV dtype, written to position seq_lens[b] - 1.
+  // Fused append (pages a multiple of 16; fp8 pools in the balanced schedule), else null:
+  // each row's newest token, [B, Hkv, 128] in the activation dtype, written to position
+  // seq_lens[b] - 1 (fp8 pools: e4m3 of x / k_scale and x / v_scale).
+  float k_scale;
   const uint8_t* k_new;
   const uint8_t* v_new;
   // Balanced schedule only: per (row, kv head) pair, {first wave, waves, T low, T high} of
@@ -589,6 +592,10 @@ struct Lines : Base {
 template <class Pager, class Raw>
 __device__ inline void ready_tile(const Pager&, Raw&, int) {}
 
+// Work of a pager between the loads of a range's first tile and those of its second.
+template <class Pager>
+__device__ inline void started(const Pager&, int) {}
+
 // The last tile of a range is computed with no further tile's loads behind it.
 template <class Pager>
 __device__ inline void last_tile(const Pager&) {}
@@ -677,6 +684,54 @@ struct Fp8Pager {
     }
   }
 };
+
+// Fp8Pager for a step that also appends each row's newest token: the write of
+// pkv_append_kv_fp8, by the wave whose tiles hold the token, before it loads that tile (no
+// other wave reads those bytes, and a wave's accesses to one address stay in order).  The
+// token's loads go out with the first page lookups; the encode runs behind the first tile's
+// loads, or before them when the token is in the first two tiles.  An append launch of its
+// own took 2-3 us of an 8-row step and its submission 3 us more of the host's time: C4 lengths
+// 26.2 -> 24.2 us per call.  Taking the encoded token into the loaded operand registers instead
+// put the encode into the tile loop and cost more than the launch.
+template <class Elem>
+struct Fp8AppendPager : Fp8Pager {
+  int lane, tail_tile;
+  bool mine;           // this wave writes the token (wave-uniform)
+  uint32_t k2, v2;     // dims 2 lane, 2 lane + 1 of the new K and V
+  long slot;           // byte offset of the token's row in the pools
+
+  __device__ Fp8AppendPager(const DecodeArgs& args, int row, int kvh, int limit, int lane_id)
+      : Fp8Pager(args, row, kvh, limit, lane_id), lane(lane_id) {
+    // limit = min(32 * t1, clamped length), so the token is in the wave's tiles when its
+    // unclamped length is `limit` (a length past the table is larger, and its append skipped).
+    int logical, in_page;
+    page_of(a, limit > 0 ? limit - 1 : 0, logical, in_page);
+    const int page = load_scalar(trow + (logical < a.max_pages ? logical : a.max_pages - 1));
+    const int raw = load_scalar(a.seq_lens + row);
+    const long src = (((long)row * a.hkv + kvh) * kD + 2 * lane) * 2;
+    k2 = *(const uint32_t*)(a.k_new + src);
+    v2 = *(const uint32_t*)(a.v_new + src);
+    mine = raw == limit && raw > 0 && (unsigned)page < (unsigned)a.num_pages;
+    slot = (long)page * page_bytes + head_bytes + (long)in_page * kD;
+    tail_tile = (limit - 1) / kTile;
+  }
+  __device__ inline void append() const {
+    if (!mine) return;
+    constexpr bool kBf16 = Elem::kPasses == 2;
+    *(uint16_t*)(const_cast<uint8_t*>(a.k_pages) + slot + 2 * lane) = (uint16_t)e4m3_pack2<kBf16>(k2, a.k_scale);
+    *(uint16_t*)(const_cast<uint8_t*>(a.v_pages) + slot + 2 * lane) = (uint16_t)e4m3_pack2<kBf16>(v2, a.v_scale);
+    asm volatile("" ::: "memory");  // the tile's loads stay behind the stores
+  }
+  __device__ inline void begin(int t0) const {
+    if (tail_tile <= t0 + 1) append();
+  }
+  __device__ inline void started(int t0) const {
+    if (tail_tile > t0 + 1) append();
+  }
+};
+
+template <class Elem>
+__device__ inline void started(const Fp8AppendPager<Elem>& pg, int t0) { pg.started(t0); }
 
 // Pager for page sizes that are not multiples of 16: a 16-token block may span pages, so
 // each token row has an address of its own.
@@ -961,6 +1016,7 @@ __device__ inline void stream_range_from(WaveState<HB, NV>& st, const Pager& pg,
     if (t0 >= t1) return;
     typename Pager::Raw ra, rb;
     pg.issue(t0, pa, ra);
+    started(pg, t0);
     int t = t0;
     for (; t + 1 < t1; t += 2) {
       pg.issue(t + 1, pb, rb);
@@ -1536,7 +1592,8 @@ __device__ inline void init_state(WaveState<HB, NV>& st) {
 // kPgLines, kPgContigLines and kPgAppendLines are kPgFast, kPgContig and kPgAppend with
 // whole-line K loads (Lines).
 enum : int { kPgGeneric = 0, kPgFast = 1, kPgContig = 2, kPgFp8 = 3, kPgAppend = 4, kPgLines = 5,
-             kPgContigLines = 6, kPgAppendLines = 7 };
+             kPgContigLines = 6, kPgAppendLines = 7, kPgFp8Append = 8 };
+constexpr bool is_fp8(int pg) { return pg == kPgFp8 || pg == kPgFp8Append; }
 
 // Streams tiles [t0, t1) of (row, kvh) into the wave state without finishing it, so that
 // several ranges can be streamed into one state (finish_state ends it).  `slab` is the
@@ -1568,6 +1625,12 @@ __device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB, NV>& st, 
     else stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
   } else if constexpr (PG == kPgFp8) {
     Fp8Pager pg(a, row, kvh, lim, lane);
+    if (have_first) stream_range_from<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, f0, f1);
+    else stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
+  } else if constexpr (PG == kPgFp8Append) {
+    if (t0 >= t1) return;
+    Fp8AppendPager<Elem> pg(a, row, kvh, lim, lane);
+    pg.begin(t0);
     if (have_first) stream_range_from<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, f0, f1);
     else stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
   } else if constexpr (PG == kPgContig) {
@@ -2109,7 +2172,7 @@ __global__ __launch_bounds__(64) void merge_kernel(MergeArgs a) {
 // (row, kv head) pair, as the builder emits it) covers each pair's tiles
 // [0, ceil(len / 32)) once, whatever its split counts; the combined work-queue op can
 // therefore stream those tiles with an equal share per wave instead of one workgroup per
-// item.  Each (row, kv head) pair with tiles is laid out as kBalPieceCost start-up
+// item.  Each (row, kv head) pair with tiles is laid out as bal_piece_cost start-up
 // positions followed by its tiles, pairs end to end (rows in order, kv heads within a
 // row), T positions in all; wave v of V takes positions [floor(v T / V), floor((v + 1) T
 // / V)), cutting pairs anywhere, and writes one partial state per pair piece that holds
@@ -2137,9 +2200,16 @@ constexpr int kBalWavesMax = 4;
 constexpr int bal_waves_per_cu(bool fp8) { return fp8 ? 4 : 2; }
 constexpr int kBalRowChunks = 4;  // lane l holds rows l + 64k, k < 4: batches up to 256
 constexpr int kBalPieceCost = 2;  // start-up positions of each (row, kv head) pair
+// fp8 pieces: a tile is half the bytes, and the pair's last piece also appends the token in an
+// appending step (the plain step keeps the same layout, so that the two agree bit for bit).  64
+// Zipf rows, G = 8, with the append: 105.2 us per call at 2, 100.9 at 3, 100.7 at 4 (102.8 with
+// an append launch); 200 rows of 20-700 tokens 25.8, 25.4 and 25.3.  Without it 4 made 8 short
+// rows 2 % slower (10.8 -> 11.1 us).
+constexpr int kBalPieceCostFp8 = 3;
+constexpr int bal_piece_cost(int pg) { return is_fp8(pg) ? kBalPieceCostFp8 : kBalPieceCost; }
 
 // The rows of a launch as one wave holds them: lane l keeps rows l + 64k (chunk k).  A
-// row weighs (kBalPieceCost + tiles) * Hkv positions, 0 without tiles; incl is the
+// row weighs (bal_piece_cost + tiles) * Hkv positions, 0 without tiles; incl is the
 // inclusive prefix of weights in row order
 // (rows past the batch weigh 0, so their prefix is the total).  The four chunks are
 // separate registers, never an array, so that selecting one by a run-time chunk index
@@ -2181,12 +2251,13 @@ __device__ inline long read_lane64(long x, int src) {
 }
 
 // One chunk: the clamped length of row lane + 64k and its inclusive prefix (carry in/out).
+template <int COST>
 __device__ inline void row_chunk(const DecodeArgs& a, int lane, int k, int raw, int& len,
                                  long& incl, long& carry) {
   const int r = lane + 64 * k;
   len = r < a.batch ? clamp_length(a, raw) : 0;
   const int tiles = ceil_tiles(len);
-  incl = wave_incl_scan(tiles > 0 ? (long)(tiles + kBalPieceCost) * a.hkv : 0, lane) + carry;
+  incl = wave_incl_scan(tiles > 0 ? (long)(tiles + COST) * a.hkv : 0, lane) + carry;
   carry = read_lane64(incl, 63);
 }
 
@@ -2209,24 +2280,26 @@ __device__ inline RowInts load_row_ints(const int32_t* p, int n, int lane, int s
                  (int)__builtin_amdgcn_raw_buffer_load_b32(r, o + 768, 0, 0)};
 }
 
+template <int COST>
 __device__ inline void row_table_from(const DecodeArgs& a, int lane, const RowInts& raw,
                                       RowTable& t) {
   const int raw0 = raw.v0, raw1 = raw.v1, raw2 = raw.v2, raw3 = raw.v3;
   // Chunks past the batch hold no row: their prefix is the total.
   long carry = 0;
-  row_chunk(a, lane, 0, raw0, t.len0, t.incl0, carry);
+  row_chunk<COST>(a, lane, 0, raw0, t.len0, t.incl0, carry);
   t.len1 = t.len2 = t.len3 = 0;
-  if (a.batch > 64) row_chunk(a, lane, 1, raw1, t.len1, t.incl1, carry);
-  if (a.batch > 128) row_chunk(a, lane, 2, raw2, t.len2, t.incl2, carry);
-  if (a.batch > 192) row_chunk(a, lane, 3, raw3, t.len3, t.incl3, carry);
+  if (a.batch > 64) row_chunk<COST>(a, lane, 1, raw1, t.len1, t.incl1, carry);
+  if (a.batch > 128) row_chunk<COST>(a, lane, 2, raw2, t.len2, t.incl2, carry);
+  if (a.batch > 192) row_chunk<COST>(a, lane, 3, raw3, t.len3, t.incl3, carry);
   if (a.batch <= 64) t.incl1 = carry;
   if (a.batch <= 128) t.incl2 = carry;
   if (a.batch <= 192) t.incl3 = carry;
   t.total = carry;
 }
 
+template <int COST>
 __device__ inline void row_table(const DecodeArgs& a, int lane, RowTable& t) {
-  row_table_from(a, lane, load_row_ints(a.seq_lens, a.batch, lane), t);
+  row_table_from<COST>(a, lane, load_row_ints(a.seq_lens, a.batch, lane), t);
 }
 
 // Length and inclusive prefix of row r (wave-uniform r): each chunk's value at lane r % 64
@@ -2370,9 +2443,10 @@ __device__ inline bool check_queue_part(const DecodeArgs& a, const RowTable& t, 
 // One workgroup of bal_waves_per_cu independent waves per CU (the launch asks for enough
 // LDS that no two share a CU).
 template <class Elem, int PG>
-__global__ __launch_bounds__(bal_waves_per_cu(PG == kPgFp8) * 64) __attribute__((amdgpu_waves_per_eu(1)))
+__global__ __launch_bounds__(bal_waves_per_cu(is_fp8(PG)) * 64) __attribute__((amdgpu_waves_per_eu(1)))
 void balanced_decode_kernel(DecodeArgs a) {
-  constexpr int kWaves = bal_waves_per_cu(PG == kPgFp8);
+  constexpr int kWaves = bal_waves_per_cu(is_fp8(PG));
+  constexpr int kCost = bal_piece_cost(PG);
   extern __shared__ int32_t bal_lds[];  // wave 0: the row table of the queue check
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
@@ -2390,11 +2464,11 @@ void balanced_decode_kernel(DecodeArgs a) {
     const RowInts so1 = load_row_ints(a.split_offsets, a.batch + 1, lane, 1);
     const int so_last = load_vector_deferred(a.split_offsets + a.batch);
     const ItemLane lead = load_item_lane(a, items > 0 ? item0 : a.num_tasks, lane);
-    row_table_from(a, lane, lens, t);
+    row_table_from<kCost>(a, lane, lens, t);
     const bool ok = check_queue_part(a, t, so0, so1, uniform(so_last), bal_lds, lead, item0, items, lane);
     if (lane == 0) a.bal_flags[blockIdx.x] = ok ? 1 : 0;
   } else {
-    row_table(a, lane, t);
+    row_table<kCost>(a, lane, t);
   }
   const long T = t.total;
   long x = v * T / V;
@@ -2404,13 +2478,13 @@ void balanced_decode_kernel(DecodeArgs a) {
     const int r = uniform(table_row(t, x));  // a row with tiles: others hold no position
     const int len = uniform(table_len(t, r));
     const int tiles = ceil_tiles(len);
-    const long span = tiles + kBalPieceCost;  // positions of each of the row's pairs
+    const long span = tiles + kCost;  // positions of each of the row's pairs
     const long off = x - (table_incl(t, r) - span * a.hkv);
     const int kvh = uniform((int)(off / span));
     const long pair0 = x - off + kvh * span;  // first position of pair (r, kvh)
     const long e = x - pair0;                 // 0 <= e < span
-    const int t0 = uniform((int)(e > kBalPieceCost ? e - kBalPieceCost : 0));
-    const long lim = x1 - pair0 - kBalPieceCost;  // tiles of the pair within this wave
+    const int t0 = uniform((int)(e > kCost ? e - kCost : 0));
+    const long lim = x1 - pair0 - kCost;  // tiles of the pair within this wave
     const int t1 = uniform(lim < tiles ? (int)(lim > 0 ? lim : 0) : tiles);
     if (t1 <= t0) break;  // the range ends among the pair's start-up positions
     // The query row is requested first and waited for only at the Q loads; the first two
@@ -2425,12 +2499,12 @@ void balanced_decode_kernel(DecodeArgs a) {
     }
     const int qh0 = kvh * G;
     u32x4 qf[1][4];
-    load_q<1, PG == kPgFp8>(a, q_loaded, r, qh0, lane, qf);
+    load_q<1, is_fp8(PG)>(a, q_loaded, r, qh0, lane, qf);
     if (t0 == 0) {
       // The wave that holds the pair's first tile records the waves its tiles span (the
-      // last tile, pair0 + kBalPieceCost + tiles - 1, lies in wave ceil((x + 1) V / T) - 1)
+      // last tile, pair0 + kCost + tiles - 1, lies in wave ceil((x + 1) V / T) - 1)
       // while its first loads are in flight: the merge then needs no row table.
-      const long vb = ((pair0 + kBalPieceCost + tiles) * V + T - 1) / T - 1;
+      const long vb = ((pair0 + kCost + tiles) * V + T - 1) / T - 1;
       if (lane == 0)
         *(u32x4*)(a.bal_plan + ((long)r * a.hkv + kvh) * 4) =
             u32x4{(uint32_t)v, (uint32_t)(vb - v + 1), (uint32_t)T, (uint32_t)(T >> 32)};
@@ -2441,7 +2515,7 @@ void balanced_decode_kernel(DecodeArgs a) {
     const long group = (long)r * a.hkv + kvh + v;
     const Dest d{a.part_m, a.part_l, a.part_acc, group * G, 1, false};
     write_wave_state<Elem, 1, false>(a, st, qh0, 0, d, lane);
-    x = pair0 + kBalPieceCost + t1;
+    x = pair0 + kCost + t1;
   }
 
 }
@@ -3022,6 +3096,7 @@ int check_quant(const Geometry& g, const KvQuant& kq) {
 void apply_quant(DecodeArgs& a, const KvQuant& kq) {
   a.kv_fp8 = kq.fp8 ? 1 : 0;
   a.score_scale = kScaleLog2 * kq.k_scale;
+  a.k_scale = kq.k_scale;
   a.v_scale = kq.v_scale;
 }
 
@@ -3032,21 +3107,28 @@ struct NewToken {
 };
 
 // The fused append of the *_append ops.  2-byte pools with pages that are multiples of
-// 16 take the new token inside the decode (AppendPager).  Other page sizes, and fp8
-// pools, run the append kernel first on the same stream: an in-decode fp8 variant (the
-// e4m3 encode on the reloaded lanes) measured slower than the two launches.
+// 16 take the new token inside the decode (AppendPager), and so do fp8 pools in the balanced
+// schedule (Fp8AppendPager).  Other page sizes, and fp8 pools elsewhere, run the append
+// kernel first on the same stream.
 // check_new_token validates the arguments without launching anything; apply_new_token
 // (after apply_quant and after every other check of the op) launches or wires the append.
 int check_new_token(const DecodeArgs& a, const NewToken& nt) {
   if (!nt.k && !nt.v) return PKV_OK;
   if (!nt.k || !nt.v) return fail(PKV_ERR_INVALID_ARGUMENT, "k_new and v_new must both be set");
   if (!a.seq_lens) return fail(PKV_ERR_INVALID_ARGUMENT, "the fused append needs seq_lens");
+  if (a.kv_fp8 && !(a.k_scale > 0.f && a.v_scale > 0.f && std::isfinite(a.k_scale) && std::isfinite(a.v_scale)))
+    return fail(PKV_ERR_INVALID_ARGUMENT, "append: k_scale and v_scale must be finite and positive");
   return PKV_OK;
 }
 
 int apply_new_token(const Geometry& g, DecodeArgs& a, const NewToken& nt, const KvQuant& kq,
-                    hipStream_t stream) {
+                    hipStream_t stream, bool balanced = false) {
   if (!nt.k && !nt.v) return PKV_OK;
+  if (a.kv_fp8 && balanced) {
+    a.k_new = (const uint8_t*)nt.k;
+    a.v_new = (const uint8_t*)nt.v;
+    return PKV_OK;
+  }
   if (a.kv_fp8)
     return pkv_append_kv_fp8(nt.k, nt.v, const_cast<uint8_t*>(a.k_pages),
                              const_cast<uint8_t*>(a.v_pages), a.block_table, a.seq_lens, g.batch,
@@ -3264,7 +3346,7 @@ int run_workqueue(const QueueCall& c, int32_t fused_merge, hipStream_t stream, c
   const int waves = balanced_waves(c.g, c.ws_bytes, fused_merge, kq.fp8);
   // Every argument is checked (the workspace by check_queue): the append may now run.
   if (stages & 1) {
-    st = apply_new_token(c.g, a, nt, kq, stream);
+    st = apply_new_token(c.g, a, nt, kq, stream, waves > 0);
     if (st != PKV_OK) return st;
   }
   if (waves > 0) {
@@ -3283,7 +3365,10 @@ int run_workqueue(const QueueCall& c, int32_t fused_merge, hipStream_t stream, c
       const size_t lds = 96 * 1024;
       const int grid = check_wgs;
       const bool bf = c.g.dtype == PKV_DTYPE_BF16;
-      if (a.kv_fp8) {
+      if (a.kv_fp8 && a.k_new) {
+        if (bf) balanced_decode_kernel<BFloat, kPgFp8Append><<<grid, wg_waves * 64, lds, stream>>>(a);
+        else balanced_decode_kernel<Half, kPgFp8Append><<<grid, wg_waves * 64, lds, stream>>>(a);
+      } else if (a.kv_fp8) {
         if (bf) balanced_decode_kernel<BFloat, kPgFp8><<<grid, wg_waves * 64, lds, stream>>>(a);
         else balanced_decode_kernel<Half, kPgFp8><<<grid, wg_waves * 64, lds, stream>>>(a);
       } else if (a.k_new) {
