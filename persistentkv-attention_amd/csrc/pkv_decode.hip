@@ -838,6 +838,56 @@ __device__ inline void ready_tile(const GenericPager& pg, TileRegs& r, int tile)
   }
 }
 
+// GenericPager with whole-line K through LDS and slices of the output dims, as Lines, for
+// launches of at most half the CUs in units.  K and V take the same eight rows per lane: instruction j of a
+// block writes rows 4g + j, so that row r of the slab lies at 1 KB x (r % 4) + 256 B x (r / 4).
+// One 2k row without a workspace, pages of 24 (8 units): 34.0 -> 17.7 us per call.  Undivided
+// units are better off without it (256 units of 16 rows of 100-6000 tokens, pages of 8, G = 8:
+// 31.0 against 31.65 us): their tiles' address work, not the CU's requests, bounds them.
+template <int NV>
+struct GenericLines : GenericPager {
+  using Raw = LineTile<NV>;
+  uint8_t* slab;
+  int slice;
+
+  __device__ GenericLines(const DecodeArgs& args, int row, int kvh, int limit, int lane_id, uint8_t* s,
+                          int slice_)
+      : GenericPager(args, row, kvh, limit, lane_id), slab(s), slice(slice_) {}
+  __device__ inline void issue(int tile, const Pages& p, Raw& r) const {
+    const int c = lane & 15, g = lane >> 4;
+    uint8_t* sb = slab + (tile & 1) * kSlabBytes;
+    asm volatile("" ::: "memory");  // K loads, then V loads, as in Lines
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(kbase + (uint64_t)p.v[j] * (kD * 2) +
+                                                          ((c ^ (4 * g + (j & 3))) * 16)),
+          (__attribute__((address_space(3))) void*)(sb + j * 1024), 16, 0, NV < 8 ? 0 : kKvLoadPolicy);
+    asm volatile("" ::: "memory");
+    const uint8_t* vdims = vbase + (slice * 16 * NV + c * NV) * 2;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      r.v[j] = __builtin_nontemporal_load(
+          (const __attribute__((address_space(1))) typename DimsOf<NV>::Type*)(vdims + (uint64_t)p.v[j] * (kD * 2)));
+    r.new_row = -1;
+    r.rd = sb + (c & 3) * 1024 + (c >> 2) * 256;
+    r.col = g ^ c;
+    asm volatile("" ::: "memory");
+  }
+};
+template <int NV>
+__device__ inline void last_tile(const GenericLines<NV>&) {
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+}
+// As Lines: at least 24 loads (and the table loads) were issued after the tile's K rows.
+template <int NV>
+__device__ inline void ready_tile(const GenericLines<NV>& pg, LineTile<NV>& r, int tile) {
+  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    r.v[j] &= tile * kTile + v_slot_token(pg.lane >> 4, j) < pg.lim ? ~0u : 0u;
+}
+
 // ---------------------------------------------------------------------------------
 // Per-wave streaming state and tile step.
 //
@@ -1040,7 +1090,7 @@ template <class Elem, int HB, class Pager, int DEPTH = HB, int NV = 8>
 __device__ inline void stream_range(WaveState<HB, NV>& st, const Pager& pg, const u32x4 (&qf)[HB][4],
                                     int t0, int t1, int lim, int lane, float qk) {
   if (t0 >= t1) return;
-  if constexpr (std::is_same_v<Pager, GenericPager>) pg.begin(t0);
+  if constexpr (std::is_base_of_v<GenericPager, Pager>) pg.begin(t0);
   const typename Pager::Pages first = pg.lookup(t0);
   stream_range_from<Elem, HB, Pager, DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, first,
                                             pg.lookup(t0 + 1));
@@ -1589,10 +1639,10 @@ __device__ inline void init_state(WaveState<HB, NV>& st) {
 
 // K/V addressing of a launch: paged with 16-token-aligned pages, paged with any page
 // size, or contiguous.
-// kPgLines, kPgContigLines and kPgAppendLines are kPgFast, kPgContig and kPgAppend with
-// whole-line K loads (Lines).
+// kPgLines, kPgContigLines, kPgAppendLines and kPgGenericLines are kPgFast, kPgContig,
+// kPgAppend and kPgGeneric with whole-line K loads (Lines, GenericLines).
 enum : int { kPgGeneric = 0, kPgFast = 1, kPgContig = 2, kPgFp8 = 3, kPgAppend = 4, kPgLines = 5,
-             kPgContigLines = 6, kPgAppendLines = 7, kPgFp8Append = 8 };
+             kPgContigLines = 6, kPgAppendLines = 7, kPgFp8Append = 8, kPgGenericLines = 9 };
 constexpr bool is_fp8(int pg) { return pg == kPgFp8 || pg == kPgFp8Append; }
 
 // Streams tiles [t0, t1) of (row, kvh) into the wave state without finishing it, so that
@@ -1614,6 +1664,11 @@ __device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB, NV>& st, 
     stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
     // The loop's last loads (the tile after the range, which reads nothing) still write
     // the slab; they are done before the LDS is used for the combine or the workgroup ends.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else if constexpr (PG == kPgGenericLines) {
+    static_assert(DEPTH == 2, "two slabs per wave");
+    GenericLines<NV> pg(a, row, kvh, lim, lane, slab, slice);
+    stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   } else if constexpr (PG == kPgFast) {
     FastPager pg(a, row, kvh, lim, lane);
@@ -1957,7 +2012,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((HB == 
 void decode_kernel(DecodeArgs a) {
   constexpr int kWaves = NW;
   constexpr int kThreads = NW * 64;
-  constexpr bool kLines = PG == kPgLines || PG == kPgContigLines || PG == kPgAppendLines;
+  constexpr bool kLines =
+      PG == kPgLines || PG == kPgContigLines || PG == kPgAppendLines || PG == kPgGenericLines;
   // The whole-line pagers' slabs share the LDS with the combine, which starts with a
   // barrier; the barrier-free combine would write it while other waves still stream.
   static_assert(!(kLines && ASYNC), "whole-line K needs the barrier combine");
@@ -2873,7 +2929,7 @@ template <class Elem, int PG, int MODE>
 hipError_t launch_lines(const DecodeArgs& a, int units, hipStream_t stream) {
   if (4 * units <= cu_count()) launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
   else if (2 * units <= cu_count()) launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
-  else launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
+  else if constexpr (PG != kPgGenericLines) launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
   return hipGetLastError();
 }
 
@@ -2887,6 +2943,7 @@ hipError_t launch_layout(const DecodeArgs& a, int grid, hipStream_t stream) {
       if (!a.block_table) return launch_lines<Elem, kPgContigLines, MODE>(a, grid, stream);
       if (a.k_new) return launch_lines<Elem, kPgAppendLines, MODE>(a, grid, stream);  // pages % 16 == 0
       if (a.page_size % 16 == 0) return launch_lines<Elem, kPgLines, MODE>(a, grid, stream);
+      if (2 * grid <= cu_count()) return launch_lines<Elem, kPgGenericLines, MODE>(a, grid, stream);
     }
   }
   if constexpr (MODE != kQueue) {

@@ -60,3 +60,21 @@ def test_work_queue(gpu, ext, page, hq):
         t("seq_lens"), t("work_items"), t("split_offsets"), counters, t("q_indices"),
         t("out_indices"), out, ws, meta["bucket_length"], page, meta["total_partial_slots"], False)
     assert_parity(out, ref)
+
+
+@pytest.mark.parametrize("page", [1, 8, 24, 100])
+@pytest.mark.parametrize("lengths,hq,hkv,splits", [
+    ([2000, 0, 33, 1555], 12, 3, 1),   # 12 units: slices of 32 dims
+    ([700, 1, 64, 640, 513] * 4, 20, 5, 1),  # 100 units: slices of 64 dims
+    ([4000, 97], 32, 8, 4)])           # 64 units, split
+def test_few_units(gpu, ext, page, lengths, hq, hkv, splits):
+    """Launches that share the CUs out by output dims (at most half as many units as CUs)."""
+    dtype = torch.bfloat16 if page == 8 else torch.float16
+    case, ref = _poisoned(page, hq, hkv, dtype, lengths, seed=page + splits)
+    b = len(lengths)
+    out = torch.empty(b, hq, 128, dtype=dtype, device=gpu)
+    ws = torch.empty(b * hq * splits * 130 if splits > 1 else 0, device=gpu)
+    ext.paged_attention_masked(case.q.to(gpu), case.k_pages.to(gpu), case.v_pages.to(gpu),
+                               case.block_table.to(gpu), case.seq_lens.to(gpu), out, ws,
+                               max(lengths), page, splits)
+    assert_parity(out, ref)
