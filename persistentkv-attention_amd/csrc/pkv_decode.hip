@@ -1,11 +1,11 @@
 // pkv_decode.hip — paged GQA decode attention for MI355X (gfx950, CDNA4).
 //
-// One workgroup (8 wave64s when G <= 16, 4 when G > 16) owns one unit of work: a
+// One workgroup (2 to 8 wave64s, by launch shape) owns one unit of work: a
 // (row, kv head) pair and a range of 32-token tiles.  The unit is a whole row (direct
 // op), one sequence split of a row (grid-split ops) or one compact work item (work-queue
 // op).  The waves stream disjoint sub-ranges of the unit's tiles, so one K/V fetch from
 // HBM serves all G query heads of the KV group, then combine their online-softmax states
-// through LDS.  K/V come from paged pools (fp16 / bf16, or fp8 e4m3 unpacked exactly in
+// through LDS.  (Few-unit launches share a unit's output dims out over 2 or 4 workgroups.)  K/V come from paged pools (fp16 / bf16, or fp8 e4m3 unpacked exactly in
 // registers) or from the contiguous [B, Hkv, N, 128] layout.
 //
 // Per wave and 32-token tile:
@@ -45,7 +45,6 @@ namespace pkv {
 
 constexpr int kD = 128;              // head dim (cuh:26)
 constexpr int kTile = 32;            // work-item tile in tokens (cuh:28)
-constexpr int kMaxWaves = 8;         // waves per workgroup: 4 or 8 (template NW)
 constexpr uint32_t kRsrcWord3 = 0x00020000u;  // raw buffer, 32-bit data format (gfx9 family)
 // Cache policy of the K/V page loads: non-temporal (the buffer instructions' nt bit).
 // Every K/V byte is read once per launch, so keeping it out of the caches leaves L2 to
