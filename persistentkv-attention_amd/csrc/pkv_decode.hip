@@ -2924,11 +2924,35 @@ void launch_slices(const DecodeArgs& a, int units, hipStream_t stream) {
   decode_kernel<Elem, 1, PG, MODE, NW, false, 2, false, NV><<<grid, dim3(NW * 64), lds, stream>>>(u);
 }
 
+// Whether the call's output shares memory with rows that the decode reads: q (an in-place
+// call) or the new tokens.  A unit's workgroup reads its rows before it writes its output, so
+// undivided units take such calls; a slice may start after another slice of its unit has
+// written.
+bool output_shares_input(const DecodeArgs& a) {
+  const auto shares = [&](const uint8_t* p, size_t rows) {
+    const size_t n = rows * kD * 2, out_n = (size_t)a.out_rows * a.hq * kD * 2;
+    return p && p < a.out + out_n && a.out < p + n;
+  };
+  const size_t tokens = (size_t)a.batch * a.hkv;
+  return shares(a.q, (size_t)a.q_rows * a.hq) || shares(a.k_new, tokens) || shares(a.v_new, tokens);
+}
+
+// The workgroups that take one unit of a whole-line launch (1: undivided).  A split launch
+// writes the workspace, and its merge the output.
+int line_slices(const DecodeArgs& a, int mode, int units) {
+  if (2 * units > cu_count() || (mode == kDirect && output_shares_input(a))) return 1;
+  return 4 * units <= cu_count() ? 4 : 2;
+}
+
 template <class Elem, int PG, int MODE>
-hipError_t launch_lines(const DecodeArgs& a, int units, hipStream_t stream) {
-  if (4 * units <= cu_count()) launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
-  else if (2 * units <= cu_count()) launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
-  else if constexpr (PG != kPgGenericLines) launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
+hipError_t launch_lines(const DecodeArgs& a, int units, int slices, hipStream_t stream) {
+  if (slices == 4) launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
+  else if (slices == 2) launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
+  else if constexpr (PG != kPgGenericLines) {
+    // Few units undivided: the eight waves of the slices, whose results are the same bits.
+    if (MODE == kDirect && 2 * units <= cu_count()) launch_slices<Elem, PG, kDirect, 8, 8>(a, units, stream);
+    else launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
+  }
   return hipGetLastError();
 }
 
@@ -2939,10 +2963,11 @@ hipError_t launch_layout(const DecodeArgs& a, int grid, hipStream_t stream) {
     const int row_tiles = (a.context + kTile - 1) / kTile;
     const int unit_tiles = MODE == kSplit ? row_tiles / a.num_splits : row_tiles;
     if (!a.kv_fp8 && use_lines(MODE, grid, unit_tiles, a.seq_lens && a.batch > 1)) {
-      if (!a.block_table) return launch_lines<Elem, kPgContigLines, MODE>(a, grid, stream);
-      if (a.k_new) return launch_lines<Elem, kPgAppendLines, MODE>(a, grid, stream);  // pages % 16 == 0
-      if (a.page_size % 16 == 0) return launch_lines<Elem, kPgLines, MODE>(a, grid, stream);
-      if (2 * grid <= cu_count()) return launch_lines<Elem, kPgGenericLines, MODE>(a, grid, stream);
+      const int slices = line_slices(a, MODE, grid);
+      if (!a.block_table) return launch_lines<Elem, kPgContigLines, MODE>(a, grid, slices, stream);
+      if (a.k_new) return launch_lines<Elem, kPgAppendLines, MODE>(a, grid, slices, stream);  // pages % 16 == 0
+      if (a.page_size % 16 == 0) return launch_lines<Elem, kPgLines, MODE>(a, grid, slices, stream);
+      if (slices > 1) return launch_lines<Elem, kPgGenericLines, MODE>(a, grid, slices, stream);
     }
   }
   if constexpr (MODE != kQueue) {
