@@ -483,8 +483,12 @@ struct ContigPager {
 //     an instruction writes the 16 bytes at slab offset 16 i): it costs no registers, and a
 //     wave keeps two tiles in flight;
 //   - each slice reads only its dims of V (2 NV bytes per lane and token row);
-//   - the slices of a unit run on one XCD in step, so that K, read by each of them, comes
-//     from HBM once (K keeps the default cache policy; each V byte is read by one slice).
+//   - the slices of a unit run on one XCD in step, so that what several of them read comes
+//     from beyond the L2 once: K, and with 32 dims V too, whose lines (64 dims) two slices
+//     share, keep the default cache policy.  With V streamed (nontemporal) at 32 dims, each
+//     line was fetched twice, which showed where K/V came from the Infinity Cache: 64 units
+//     of 4k tokens just written took 42.2 us, 32.0 undivided, and take 25.9; 8 units of 2k
+//     14.2, 14.2 and 11.6.  From HBM: 64 of 4k 34.2 -> 33.2, 8 of 2k 15.96 -> 16.19.
 // A slab holds a tile's two 16-token blocks, 16 rows x 256 B each, with
 // 16-byte column `col` of row `row` at position col ^ row: instruction j of a block
 // writes rows 4j .. 4j + 3 (lane (c, g): row 4j + g, position c, so it loads column
@@ -500,6 +504,9 @@ template <> struct DimsOf<8> {
   __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kKvLoadPolicy);
   }
+  __device__ static inline Type load(const uint8_t* p) {
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) Type*)p);
+  }
   __device__ static inline uint32_t word(const Type& v, int i) { return v[i]; }
 };
 template <> struct DimsOf<4> {
@@ -507,12 +514,18 @@ template <> struct DimsOf<4> {
   __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kKvLoadPolicy);
   }
+  __device__ static inline Type load(const uint8_t* p) {
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) Type*)p);
+  }
   __device__ static inline uint32_t word(const Type& v, int i) { return v[i]; }
 };
 template <> struct DimsOf<2> {
   using Type = uint32_t;
   __device__ static inline Type load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kKvLoadPolicy);
+    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);  // half a line (see Lines)
+  }
+  __device__ static inline Type load(const uint8_t* p) {
+    return *(const __attribute__((address_space(1))) Type*)p;
   }
   __device__ static inline uint32_t word(const Type& v, int) { return v; }
 };
@@ -866,8 +879,7 @@ struct GenericLines : GenericPager {
     const uint8_t* vdims = vbase + (slice * 16 * NV + c * NV) * 2;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      r.v[j] = __builtin_nontemporal_load(
-          (const __attribute__((address_space(1))) typename DimsOf<NV>::Type*)(vdims + (uint64_t)p.v[j] * (kD * 2)));
+      r.v[j] = DimsOf<NV>::load(vdims + (uint64_t)p.v[j] * (kD * 2));
     r.new_row = -1;
     r.rd = sb + (c & 3) * 1024 + (c >> 2) * 256;
     r.col = g ^ c;
