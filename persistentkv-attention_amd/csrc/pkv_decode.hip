@@ -1694,6 +1694,9 @@ __device__ inline void stream_tiles(const DecodeArgs& a, WaveState<HB, NV>& st, 
     if (have_first) stream_range_from<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk, f0, f1);
     else stream_range<Elem, HB, decltype(pg), DEPTH>(st, pg, qf, t0, t1, lim, lane, qk);
   } else if constexpr (PG == kPgFp8Append) {
+    // A token past the range's first two tiles is written by started(), which the loop of one
+    // tile in flight does not call.
+    static_assert(DEPTH == 2, "the append of a later tile's token needs the two-tile loop");
     if (t0 >= t1) return;
     Fp8AppendPager<Elem> pg(a, row, kvh, lim, lane);
     pg.begin(t0);
