@@ -2961,12 +2961,17 @@ int line_slices(const DecodeArgs& a, int mode, int units) {
 
 template <class Elem, int PG, int MODE>
 hipError_t launch_lines(const DecodeArgs& a, int units, int slices, hipStream_t stream) {
-  if (slices == 4) launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
-  else if (slices == 2) launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
-  else if constexpr (PG != kPgGenericLines) {
+  if (slices == 4) {
+    launch_slices<Elem, PG, MODE, 2, 8>(a, units, stream);
+  } else if (slices == 2) {
+    launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
+  } else if constexpr (PG == kPgGenericLines) {
+    return hipErrorInvalidConfiguration;  // odd page sizes have no undivided form
+  } else if (MODE == kDirect && 2 * units <= cu_count()) {
     // Few units undivided: the eight waves of the slices, whose results are the same bits.
-    if (MODE == kDirect && 2 * units <= cu_count()) launch_slices<Elem, PG, kDirect, 8, 8>(a, units, stream);
-    else launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
+    launch_slices<Elem, PG, kDirect, 8, 8>(a, units, stream);
+  } else {
+    launch_slices<Elem, PG, MODE, 8, 3>(a, units, stream);
   }
   return hipGetLastError();
 }
