@@ -2925,7 +2925,7 @@ bool use_lines(int mode, int units, int unit_tiles, bool ragged) {
   }();
   if (mode == kQueue || forced == 0) return false;
   const int cus = cu_count();
-  return forced == 1 || (unit_tiles >= 16 && (8 * units <= 7 * cus || (ragged && units <= cus)));
+  return forced == 1 || (unit_tiles >= 16 && (units <= 7 * cus / 8 || (ragged && units <= cus)));
 }
 
 template <class Elem, int PG, int MODE, int NV, int NW>
@@ -2955,8 +2955,8 @@ bool output_shares_input(const DecodeArgs& a) {
 // The workgroups that take one unit of a whole-line launch (1: undivided).  A split launch
 // writes the workspace, and its merge the output.
 int line_slices(const DecodeArgs& a, int mode, int units) {
-  if (2 * units > cu_count() || (mode == kDirect && output_shares_input(a))) return 1;
-  return 4 * units <= cu_count() ? 4 : 2;
+  if (units > cu_count() / 2 || (mode == kDirect && output_shares_input(a))) return 1;
+  return units <= cu_count() / 4 ? 4 : 2;
 }
 
 template <class Elem, int PG, int MODE>
@@ -2967,7 +2967,7 @@ hipError_t launch_lines(const DecodeArgs& a, int units, int slices, hipStream_t 
     launch_slices<Elem, PG, MODE, 4, 8>(a, units, stream);
   } else if constexpr (PG == kPgGenericLines) {
     return hipErrorInvalidConfiguration;  // odd page sizes have no undivided form
-  } else if (MODE == kDirect && 2 * units <= cu_count()) {
+  } else if (MODE == kDirect && units <= cu_count() / 2) {
     // Few units undivided: the eight waves of the slices, whose results are the same bits.
     launch_slices<Elem, PG, kDirect, 8, 8>(a, units, stream);
   } else {
