@@ -1222,18 +1222,6 @@ __device__ inline void put_f32x4(float* p, f32x4 v, bool coherent) {
     *(f32x4*)p = v;
   }
 }
-template <bool COHERENT>
-__device__ inline float get_f32(const float* p) {
-  if (COHERENT) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return *p;
-}
-__device__ inline f32x4 get_f32x4_coherent(const float* p) {
-  const f32x2 lo = __builtin_bit_cast(f32x2, __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT));
-  const f32x2 hi = __builtin_bit_cast(f32x2, __hip_atomic_load((const uint64_t*)p + 1, __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT));
-  return f32x4{lo[0], lo[1], hi[0], hi[1]};
-}
 // Waits until every memory access this wave issued has completed.
 
 // Neutral partial state of an empty split (cuh:340-363): m = -FLT_MAX, l = 0, acc = 0.
@@ -1379,6 +1367,10 @@ struct SlotChunk {
 
 // Loads slots [c0, c0 + n) through buffer descriptors that cover exactly their states (n >=
 // 1): lanes past them read zeros, and when `enable` is false the descriptors cover nothing.
+// AUX: the loads' cache policy (kAgentLoad for states written by other workgroups of the
+// launch).
+constexpr int kAgentLoad = 16;  // sc1: agent scope, as a relaxed agent-scope atomic load
+template <int AUX = 0>
 __device__ inline void load_chunk_if(SlotChunk& c, const float* pm, const float* pl, const float* pacc,
                                      long base, long stride, int c0, int n, int lane, bool enable) {
   n = uniform(n);
@@ -1391,34 +1383,25 @@ __device__ inline void load_chunk_if(SlotChunk& c, const float* pm, const float*
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(pacc + base * kD), (short)0, uniform(span * kD * 4), kRsrcWord3);
   const int s_lane = fold_state(lane) < n ? fold_state(lane) : n - 1;
-  c.ms = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (int)(s_lane * stride * 4), 0, 0));
-  c.ls = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, (int)(s_lane * stride * 4), 0, 0));
+  c.ms = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (int)(s_lane * stride * 4), 0, AUX));
+  c.ls = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rl, (int)(s_lane * stride * 4), 0, AUX));
   const int pair = (int)(2 * stride) * (kD * 4);
   const int off = (int)((lane >> 5) * stride) * (kD * 4) + (lane & 31) * 16;
 #pragma unroll
   for (int i = 0; i < kMergeChunk / 2; ++i)
-    c.v[i] = 2 * i < n ? __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, off + i * pair, 0, 0))
+    c.v[i] = 2 * i < n ? __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, off + i * pair, 0, AUX))
                        : f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
-// The same with agent-scope loads, of states written by other workgroups of the launch.
+// The fused merge takes agent-scope loads.  As 8-byte atomic loads, each with an address and a
+// branch per lane, they took its kernels from 123 to 183 registers (fp8 K/V), and with them
+// the second workgroup of a CU: 64 Zipf rows with fp8 K/V and the fused merge 118.5 us per
+// call, 108.6 through the descriptors, 8 rows of 200-900 tokens 12.8 and 12.1.  8 bimodal
+// rows, whose few items end sooner with a CU to themselves, 70.0 and 74.4.
 template <bool COHERENT>
 __device__ inline void load_chunk(SlotChunk& c, const float* pm, const float* pl, const float* pacc,
                                   long base, long stride, int c0, int n, int lane) {
-  if constexpr (!COHERENT) {
-    load_chunk_if(c, pm, pl, pacc, base, stride, c0, n, lane, true);
-  } else {
-    n = uniform(n);
-    const int s_lane = c0 + (fold_state(lane) < n ? fold_state(lane) : n - 1);
-    c.ms = get_f32<true>(pm + base + (long)s_lane * stride);
-    c.ls = get_f32<true>(pl + base + (long)s_lane * stride);
-#pragma unroll
-    for (int i = 0; i < kMergeChunk / 2; ++i) {
-      const int j = 2 * i + (lane >> 5);
-      c.v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (j < n) c.v[i] = get_f32x4_coherent(pacc + (base + (long)(c0 + j) * stride) * kD + 4 * (lane & 31));
-    }
-  }
+  load_chunk_if<COHERENT ? kAgentLoad : 0>(c, pm, pl, pacc, base, stride, c0, n, lane, true);
 }
 
 // Whether slot s of a row holds a state.  In queue mode the builder leaves splits with no
