@@ -513,9 +513,10 @@ int pkv_append_kv_fp8(const void* k_new, const void* v_new, void* k_pages, void*
 /* Decode with the append fused in: the result and the pools afterwards equal
  * pkv_append_kv(k_new, v_new, ...) followed by the op without the suffix, in one decode
  * launch.  The newest token of each row (position seq_lens[b] - 1) is read from k_new /
- * v_new ([batch, num_kv_heads, 128], `dtype`) by the one wave whose tiles hold it, which
- * also writes it into the pools.  Page sizes that are not multiples of 16 run
- * pkv_append_kv first on the same stream.  (fp8 pools: the *_fp8_append entries below.)  A row's tail slot must not be read
+ * v_new ([batch, num_kv_heads, 128], `dtype`) by the waves whose tiles hold it (one, or one
+ * of each workgroup that shares the unit's output dims), one of which also writes it into
+ * the pools.  Page sizes that are not multiples of 16 run pkv_append_kv first on the same
+ * stream.  (fp8 pools: the *_fp8_append entries below.)  A row's tail slot must not be read
  * through another (row, position) of the same step (no two rows share a tail page, as
  * in any copy-on-write cache).  No counterpart in the reference (see pkv_append_kv). */
 int pkv_paged_attention_masked_append(
@@ -556,9 +557,14 @@ int pkv_paged_attention_workqueue_append(
 
 /* The fp8-K/V ops with the append: k_new / v_new are in `dtype` and stored as
  * pkv_append_kv_fp8 stores them, e4m3(clamp(x / k_scale)) and e4m3(clamp(x / v_scale)).
- * Same result as pkv_append_kv_fp8 followed by the fp8 op, which is what they run but for
- * the work-queue op's balanced schedule, whose decode writes the tokens itself (no two rows
- * may share a tail page, as above).  v_scale must be positive. */
+ * Same result as pkv_append_kv_fp8 followed by the fp8 op.  That is also what they run, two
+ * launches in stream order, in the indexed op and in the work-queue op's per-item schedule.
+ * In its balanced schedule (pkv_workqueue_schedule names the schedule of a call: it follows
+ * from the workspace size, fused_merge, G, page_size and batch) the decode writes the tokens
+ * itself, and a row's tail slot must not be read through another (row, position) of the
+ * same step, as above: of two rows that share a tail page, each may then read the other's
+ * slot before or after it is written.  Callers with shared tail pages run pkv_append_kv_fp8
+ * and the op without the suffix.  v_scale must be positive. */
 int pkv_paged_attention_indexed_fp8_append(
     const void* q_source, int32_t q_rows,
     const void* k_pages, const void* v_pages,
