@@ -477,8 +477,10 @@ struct ContigPager {
 // are shared out by output dims: 8 / NV workgroups ("slices") take one unit, each the whole
 // QK product and 16 NV of the 128 output dims, so they need no memory to meet in and a
 // launch without a workspace still uses several CUs per unit.  What one CU streams bounds
-// such a launch (35-37 GB/s with the K-operand shape, 16 rows x 64 B per instruction, 45-56
-// GB/s with whole lines), so
+// such a launch: 35-37 GB/s from HBM with the K-operand shape (16 rows x 64 B per
+// instruction); with whole lines 57-61 GB/s from HBM and 96-111 GB/s from the Infinity Cache,
+// over a 50k-token row in 1, 2 and 4 slices alike, so a unit's time follows the bytes that
+// each of its CUs moves (16, 12 and 10 KB per tile).  So
 //   - K takes whole 128-byte lines straight to LDS (buffer_load_dwordx4 ... lds: lane i of
 //     an instruction writes the 16 bytes at slab offset 16 i): it costs no registers, and a
 //     wave keeps two tiles in flight;
@@ -1070,7 +1072,8 @@ __device__ inline void stream_range_from(WaveState<HB, NV>& st, const Pager& pg,
   } else {
     // One wave per SIMD, half the waves of a CU at one block: each wave keeps two tiles
     // in flight, so the CU holds as many bytes in flight as there.  Loads of tile t1 (one
-    // past the range) cover no valid rows and read nothing.  The loop has one exit, taken
+    // past the range) cover no valid rows and read nothing (odd page sizes: the last valid
+    // row again).  The loop has one exit, taken
     // with only `ra` in flight: with a second exit between the tiles the compiler merged
     // the two into one block where `rb` may still be in flight, and waited before every
     // issue of `rb` until 5 to 13 of the 16 loads of `ra` had landed.
@@ -1222,8 +1225,6 @@ __device__ inline void put_f32x4(float* p, f32x4 v, bool coherent) {
     *(f32x4*)p = v;
   }
 }
-// Waits until every memory access this wave issued has completed.
-
 // Neutral partial state of an empty split (cuh:340-363): m = -FLT_MAX, l = 0, acc = 0.
 __device__ inline void write_neutral(const DecodeArgs& a, long state0, long state_stride,
                                      int G, int tid, int nthreads, bool coherent) {
@@ -1465,8 +1466,7 @@ __device__ inline void fold_slots_pipelined(LseAcc& acc, const float* pm, const 
 }
 
 // Wide fold of up to kWideStates states of one query head by one wave, every load in
-// flight at once (one memory round trip; a wave tracks at most 63 vector loads, so the
-// 8-byte loads of fold_slots fit 32 states per round trip).  Lanes 0-31 load the even
+// flight at once (one memory round trip; a wave tracks at most 63 vector loads).  Lanes 0-31 load the even
 // states and lanes 32-63 the odd ones with 16-byte loads (4 dims per lane): 2 states per
 // load.  Lane j holds (m, l) of states j and j + 64.  Each half accumulates its states (the
 // LseAcc layout).  States are base + s * stride, s < n (wave-uniform, 1 <= n <=
@@ -1999,7 +1999,6 @@ __device__ inline void zero_empty_rows(const DecodeArgs& a, int tid, int threads
   }
 }
 
-//
 // NV < 8: the 8 / NV workgroups of a unit each compute 16 NV of its output dims (Lines).
 // Workgroup b runs on XCD b % 8, so unit u's slices are workgroups u / 8 * 8 * slices +
 // slice * 8 + u % 8.
@@ -2883,22 +2882,27 @@ hipError_t launch_decode(const DecodeArgs& a, int grid, hipStream_t stream) {
 
 // Direct and split launches of at most one unit per CU, of at least 16 tiles each, whose
 // longest units end on CUs that stream alone: launches that leave an eighth of the CUs idle
-// or whose rows differ in length.  A lone CU moves ~512 requests (128-byte lines) per us
-// whatever is in flight, so whole-line K loads (Lines), half the requests of the K-operand
-// shape, shorten the end of the launch.
+// or whose rows differ in length.  A lone CU moves more with whole-line K loads (Lines).
 //   - At most half the CUs in units: the CUs are shared out by output dims, 4 slices of 32
-//     dims per unit up to a quarter of the CUs, else 2 of 64 (a slice's requests are its
-//     unit's K lines and a quarter or half of the V bytes).  8 waves with two tiles in
-//     flight.  One 2k row without a workspace (8 units): 15.3 us with 4 slices, 17.5 with 2,
-//     21.7 undivided; 32 units 22.7 -> 17.7 us, 64 units 23.9 -> 19.5, 128 units 26.8 -> 24.9;
+//     dims per unit up to a quarter of the CUs, else 2 of 64: 10 and 12 KB per tile and CU
+//     for the undivided 16.  8 waves with two tiles in flight.  Undivided, 2 and 4 slices, us
+//     per call, with K/V from HBM and just written (Infinity Cache):
+//         8 units of 2k tokens    21.8  18.0  16.2     14.2  12.9  11.6
+//        64 units of 2k           23.9  20.8  19.2     19.8  16.6  16.5
+//         8 units of 9k           80.9  63.9  56.2     47.1  40.6  35.5
+//        64 units of 4k           43.1  36.2  33.2     32.0  26.4  25.9
+//       128 units of 2k           26.8  24.8   -       26.9  23.6   -
 //     16 split units of an 8k row 13.4 -> 12.8 us, of a 32k row 30.3 -> 28.2.  Starting the
-//     slices of a unit a quarter of its tiles apart, for more K hits in L2: 16.2 us.
+//     slices of a unit a quarter of its tiles apart, for more K hits in L2, was slower.
 //   - More units: undivided, 3 waves with two tiles in flight.  256 units of 32 rows of
-//     16-1024 tokens 17.7 -> 14.8 us, 192 of 24 rows to 2048 30.5 -> 23.1, 136 equal ones
-//     19.0 -> 14.9, 224 equal ones 38.7 -> 37.1; 4 waves 14.98, 22.9, 15.3 and 36.8, 2 waves
-//     15.1, 24.7, 16.2 and 37.1.  256 equal units keep every CU streaming to the end and are
-//     better off with the K-operand shape (22.5 against 23.0 us), so launches without
-//     per-row lengths, or of one row, take this path only up to 7/8 of the CUs.
+//     16-1024 tokens 17.6 -> 14.4 us (just written 16.3 -> 14.8), 192 of 24 rows to 2048
+//     31.8 -> 23.8 (25.5 -> 22.4), 136 equal ones 21.7 -> 15.9, 224 equal ones 40.6 -> 38.9;
+//     2 waves, the K-operand path's split of a unit's tiles and so its bits, 14.7, 26.0, 16.5
+//     and 38.8 us, but slower than that path on just-written K/V (17.1 and 28.0).
+//     256 equal units keep every CU streaming to the end and are better off with the
+//     K-operand shape (1k tokens 22.4 against 23.0 us, 2k 44.0 against 44.4, 4k the same), so
+//     launches without per-row lengths, or of one row, take this path only up to 7/8 of the
+//     CUs; with per-row lengths the host cannot tell equal rows from others.
 // Units of 8 tiles or fewer are latency-bound and 0.2-0.4 us slower this way (the LDS round
 // trip).  PKV_LINES=0|1 forces the choice (tuning, tests).
 bool use_lines(int mode, int units, int unit_tiles, bool ragged) {
