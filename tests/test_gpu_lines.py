@@ -2,9 +2,9 @@
 
 A direct launch (num_splits == 1) with no workspace to split into, or a split launch
 whose workspace holds no sub-splits, of at most half as many units as the GPU has CUs and
-at least 16 tiles (512 tokens) per unit, runs one workgroup per unit whose K loads take
-whole 128-byte lines straight into LDS (the reference's own C1 call: one row, 8 KV heads,
-`workspace` empty).  Each case here is such a launch, against the repack + fp32 SDPA
+at least 16 tiles (512 tokens) per unit, runs 2 or 4 workgroups per unit, each with a slice
+of the output dims, whose K loads take whole 128-byte lines straight into LDS (the
+reference's own C1 call: one row, 8 KV heads, `workspace` empty).  Each case here is such a launch, against the repack + fp32 SDPA
 oracle at the parity bar (max-abs 2e-3, mean-abs 3e-4): every op with a grid launch
 (paged, masked, indexed, contiguous, the query-head baseline, the fused append), direct
 and split, fp16 and bf16, G from 1 to 16, page sizes that are multiples of 16, ragged and
